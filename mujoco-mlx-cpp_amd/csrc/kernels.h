@@ -370,7 +370,7 @@ KDEV void cross_force(const float* v, const float* f, float* r) {
 // walked two to four dependent loads (level list, parent, joint, type) at
 // 200-500 cycles each, which bound the stages between the state and the
 // solver: 37 % of a quadruped's step, 60 % of a small arm's. Per control step:
-// 16384 quadrupeds 3.12 -> 2.98 ms, 64 quadrupeds 404 -> 383 us, 16384 arms
+// 16384 quadrupeds 3.22 -> 3.07 ms, 64 quadrupeds 423 -> 399 us, 16384 arms
 // (8 dofs) 1.34 -> 1.22 ms, same bits; the humanoid's multi-joint bodies gain
 // nothing measurable.
 typedef int ki4 __attribute__((vector_size(16)));
@@ -809,7 +809,7 @@ KDEV int factor_ld(const DModel& m, const float* A, float* LD) {
 // ways. So the larger size refines (+0.04 ms of 0.81 at 517 humanoids), the
 // smaller doesn't need to. Bound by its instructions' issue, about two per pair
 // (k, j). Per control step: 16384 / 517 humanoids (implicit damping) 5.36 ->
-// 4.88 / 0.90 -> 0.84 ms, 16384 / 64 quadrupeds 2.98 -> 2.94 ms / 383 -> 373 us.
+// 4.88 / 0.90 -> 0.84 ms. Elliptic cones only (solve_in_regs).
 template <int NVM>
 KDEV int ltdl_solve_regs(int nv, const float* A, float* x) {
   float h[NVM];
@@ -861,10 +861,14 @@ KDEV int ltdl_solve_regs(int nv, const float* A, float* x) {
 KDEV int smooth_solve_regs(int nv, const float* A, float* x) {
   return nv <= 20 ? ltdl_solve_regs<20>(nv, A, x) : ltdl_solve_regs<32>(nv, A, x);
 }
-// the factor of qM itself is needed by CG's preconditioner only
-KDEV bool solve_in_regs(const DModel& m) { return m.solver == 2; }
+// Newton models with elliptic cones; the factor of qM itself is CG's
+// preconditioner, and pyramidal models keep the rounding of the level sums
+// (newton_direction says why). REGS: not the 168-VGPR kernels.
+template <bool REGS>
+KDEV bool solve_in_regs(const DModel& m) { return REGS && m.solver == 2 && m.cone != 0; }
 #else
 KDEV int smooth_solve_regs(int, const float*, float*) { return 0; }
+template <bool REGS>
 KDEV bool solve_in_regs(const DModel&) { return false; }
 #endif
 
@@ -1120,6 +1124,7 @@ KDEV float free_drag(const DModel& m, const Layout& L, const float* w, int k) {
   return kd * v[i];
 }
 
+template <bool REGS>
 KDEV int st_smooth(const DModel& m, const Layout& L, float* w) {
   float *cacc = w + L.cacc, *cfrc = w + L.cfrc;
   const float *cinert = w + L.cinert, *cvel = w + L.cvel, *cdd = w + L.cdofdot, *cdof = w + L.cdof;
@@ -1193,7 +1198,7 @@ KDEV int st_smooth(const DModel& m, const Layout& L, float* w) {
     qas[k] = s;
   }
   KSYNC();
-  if (solve_in_regs(m)) return smooth_solve_regs(m.nv, w + L.qM, qas);
+  if (solve_in_regs<REGS>(m)) return smooth_solve_regs(m.nv, w + L.qM, qas);
   solve_ld(m, w + L.qLD, qas);
   return 0;
 }
@@ -2686,7 +2691,11 @@ KDEV void grad_only(const DModel& m, const Layout& L, float* w, int nefc) {
 
 // with_grad false: forces, active flags and cost only (comparing warm-start
 // candidates), no gradient
-KDEV float cost_grad(const DModel& m, const Layout& L, float* w, int nefc, int* nchanged, bool with_grad = true) {
+// chmask (when not null): the rows whose activity changed, bit r % 64 of word
+// r / 64, for pyramidal / frictionless / limit / friction-loss rows of at most
+// 128 rows on 64 lanes (or the serial interpreter); otherwise both words ~0
+KDEV float cost_grad(const DModel& m, const Layout& L, float* w, int nefc, int* nchanged, bool with_grad = true,
+                     unsigned long long* chmask = nullptr) {
   int nv = m.nv;
   const float *Jaref = w + L.efc_Jaref, *D = w + L.efc_D;
   float *force = w + L.efc_force, *Dact = w + L.efc_Dact;
@@ -2694,7 +2703,9 @@ KDEV float cost_grad(const DModel& m, const Layout& L, float* w, int nefc, int* 
   const int* eid = iptr(w, L.efc_id);
   float part = 0.f;
   int nch = 0;
-  for (int r = LANE; r < nefc; r += WAVE) {
+  unsigned long long cm[2] = {0ull, 0ull};
+  int q = 0;
+  for (int r = LANE; r < nefc; r += WAVE, q++) {
     float x = Jaref[r], d = D[r];
     int ty = etype[r];
     if (ty == EFC_CONTACT_ELLIPTIC) continue;  // per contact, below
@@ -2709,8 +2720,17 @@ KDEV float cost_grad(const DModel& m, const Layout& L, float* w, int nefc, int* 
       if (x < 0.f) { act[r] = 1; force[r] = -d * x; part += 0.5f * d * x * x; }
       else { act[r] = 0; force[r] = 0.f; }
     }
-    nch += act[r] != old;
+    bool chg = act[r] != old;
+    nch += chg;
     Dact[r] = act[r] ? d : 0.f;
+#if WAVE == 64
+    unsigned long long b = __ballot(chg);
+    if (q < 2) cm[q] = b;
+#elif WAVE == 1
+    if (chg && r < 128) cm[r >> 6] |= 1ull << (r & 63);
+#else
+    (void)q;
+#endif
   }
   if (m.cone != 0) {
     const int* misc = reinterpret_cast<const int*>(w + L.misc);
@@ -2736,6 +2756,18 @@ KDEV float cost_grad(const DModel& m, const Layout& L, float* w, int nefc, int* 
   for (int i = LANE; i < nv; i += WAVE) part += 0.5f * (Ma[i] - qfs[i]) * (qacc[i] - qas[i]);
   float cost = wsum(part);
   *nchanged = wsumi(nch);
+  if (chmask) {
+    bool known = (WAVE == 64 || WAVE == 1) && nefc <= 128 && m.cone == 0;
+#if WAVE == 64
+    // lane 0 takes part in every round that any lane does
+    for (int k = 0; k < 2; k++) {
+      unsigned lo = __builtin_amdgcn_readlane((unsigned)cm[k], 0), hi = __builtin_amdgcn_readlane((unsigned)(cm[k] >> 32), 0);
+      cm[k] = ((unsigned long long)hi << 32) | lo;
+    }
+#endif
+    chmask[0] = known ? cm[0] : ~0ull;
+    chmask[1] = known ? cm[1] : ~0ull;
+  }
   KSYNC();
   if (with_grad) grad_only(m, L, w, nefc);
   return cost;
@@ -2843,7 +2875,7 @@ KDEV void hessian_tiles(int nv, int nrow, const float* J, const float* Dact, con
 // workspace took a latency-bound LDS phase per two columns, a separate solve
 // and, to avoid both, rank-1 updates of the stored factor for one or two
 // changed rows. Per control step, batches of 16384 / 517 humanoids (27 dofs)
-// 6.77 -> 6.17 / 1.27 -> 1.13 ms, 16384 quadrupeds (18 dofs) 3.22 -> 3.11 ms.
+// 6.77 -> 6.17 / 1.27 -> 1.13 ms. Elliptic cones only (newton_direction).
 // Two sizes, 20 and 32 dofs: h takes 40 or 64 registers.
 template <int NVM>
 KDEV int ldl_solve_regs(int nv, const float* A, const float* b, float* x) {
@@ -3105,6 +3137,75 @@ KDEV int newton_factor(const DModel& m, const Layout& L, float* w, int nefc, KPr
   return wori(bad) ? ST_NOT_PD : 0;
 }
 
+// Rank-1 changes of the factored Hessian for rows whose activity changed
+// (H += D_r J_r^T J_r for a row that became active, -= for one that left):
+// the LDL^T update of Gill, Golub, Murray and Saunders (1974, method C1) on
+// newton_factor's storage (H_ij = L_ij d_j below the diagonal, H_jj = d_j,
+// dvec = 1 / d), one column step per dof with the row's J entries in lanes.
+// Returns false (the caller factors anew) when a pivot would lose more than
+// ten digits, which a downdate of M + J^T D J should not do.
+KDEV bool newton_update(const DModel& m, const Layout& L, float* w, const unsigned long long* chmask) {
+  int nv = m.nv;
+  double* H = dptr(w, L.H);
+  double* idg = dptr(w, L.dvec);
+  const float *J = w + L.efc_J, *D = w + L.efc_D;
+  const int* act = iptr(w, L.efc_act);
+  if (chmask[0] == ~0ull && chmask[1] == ~0ull) return false;  // rows not known
+  if (WAVE > 1 && nv > WAVE) return false;  // one lane per dof below
+  for (int q = 0; q < 2; q++) {
+    unsigned long long bits = chmask[q];
+    while (bits) {
+      int r = 64 * q + __builtin_ctzll(bits);
+      bits &= bits - 1;
+      double a = act[r] ? (double)D[r] : -(double)D[r];
+#if WAVE == 64
+      double z = LANE < nv ? (double)J[r * nv + LANE] : 0.0;
+      double d = LANE < nv ? H[hx(LANE, LANE)] : 1.0, id = LANE < nv ? idg[LANE] : 1.0;
+      for (int j = 0; j < nv; j++) {
+        double p = rl_d(z, j), dj = rl_d(d, j), idj = rl_d(id, j);
+        double dn = dj + a * p * p;
+        if (!(dn > 1e-10 * dj)) return false;
+        double idn = krcp(dn), beta = p * a * idn;
+        a *= dj * idn;
+        if (LANE == j) { d = dn; id = idn; }
+        if (LANE > j && LANE < nv) {
+          double* hp = H + hx(LANE, j);
+          double lij = *hp * idj;
+          z -= p * lij;
+          lij += beta * z;
+          *hp = lij * dn;
+        }
+      }
+      if (LANE < nv) { H[hx(LANE, LANE)] = d; idg[LANE] = id; }
+      KSYNC();
+#elif WAVE == 1
+      double* z = dptr(w, L.dvec) + nv;
+      for (int i = 0; i < nv; i++) z[i] = (double)J[r * nv + i];
+      for (int j = 0; j < nv; j++) {
+        double p = z[j], dj = H[hx(j, j)], idj = idg[j];
+        double dn = dj + a * p * p;
+        if (!(dn > 1e-10 * dj)) return false;
+        double idn = krcp(dn), beta = p * a * idn;
+        a *= dj * idn;
+        for (int i = j + 1; i < nv; i++) {
+          double* hp = H + hx(i, j);
+          double lij = *hp * idj;
+          z[i] -= p * lij;
+          lij += beta * z[i];
+          *hp = lij * dn;
+        }
+        H[hx(j, j)] = dn;
+        idg[j] = idn;
+      }
+#else
+      (void)a; (void)J; (void)H; (void)idg;
+      return false;
+#endif
+    }
+  }
+  return true;
+}
+
 // Mgrad = H^-1 grad with the factor of newton_factor, in FP64; on the GPU the
 // vector is held across lanes and each column step is a readlane broadcast.
 KDEV void newton_solve(const DModel& m, const Layout& L, float* w) {
@@ -3171,41 +3272,51 @@ KDEV void newton_solve(const DModel& m, const Layout& L, float* w) {
   KSYNC();
 }
 
-// Mgrad = H^-1 grad, H = M + J^T diag(D act) J. Models of at most 32 dofs on
-// 64 lanes build, factor and solve in one pass through the registers; the
-// others factor H in the workspace when the active set changed (refactor) and
-// solve with the stored factor.
+// Mgrad = H^-1 grad, H = M + J^T diag(D act) J. Models of at most 32 dofs with
+// elliptic cones, on 64 lanes, build, factor and solve in one pass through the
+// registers. The others solve with the factor in the workspace, which takes
+// rank-1 updates for one or two rows that changed activity (chmask, dense rows)
+// and is built anew for more (refactor: in any case).
+// Why the cones decide: pyramidal models update the stored FP64 factor, elliptic
+// ones never do (their middle zone moves H at every step), so a factor built
+// from H's FP32 sums each time is what elliptic models had and pyramidal ones
+// had not. The difference is FP32 rounding of the direction, but the solver
+// stops on the FP32 difference of two costs, where rounding decides in about
+// one of 1e5 solves whether a last step is taken: built anew (and with qM's
+// solve in registers), 18 of 491520 implicitfast quadrupeds ended more than
+// 8e-4 of the RMS velocity away after 4 substeps (up to 2e-2), with the updates
+// none; of 5.6 million humanoids none either way.
+// The 168-VGPR kernels (TRI_CACHE false) have the workspace's factor only: with
+// the register routines compiled in they spill (16384 quadrupeds, which never
+// call them, 3.39 ms per control step against 3.22 without).
 template <bool TRI_CACHE>
-KDEV int newton_direction(const DModel& m, const Layout& L, float* w, int nefc, bool refactor, KProfAcc* pa) {
-#if WAVE == 64 && !MJK_BIG
-  (void)refactor;
-  int nv = m.nv, nrow = nefc;
-  if (m.cone != 0) {
-    int nr = cone_virtual_rows(m, L, w, nefc);
-    if (nr >= 0) nrow = nr;
-    else {  // the row buffer does not hold the cones' virtual rows
-      int st = newton_factor<TRI_CACHE>(m, L, w, nefc, pa);
-      newton_solve(m, L, w);
-      return st;
-    }
-  }
-  float* A = w + L.H;
-  hessian_tiles(nv, nrow, w + L.efc_J, w + L.efc_Dact, w + L.qM, [&](int i, int j, float v) {
-    A[i * nv + j] = v;
-    A[j * nv + i] = v;
-  });
-  KSYNC();
-  KPROF_MARK(pa, KP_SPARE);
-  int bad = nv <= 20 ? ldl_solve_regs<20>(nv, A, w + L.grad, w + L.Mgrad) : ldl_solve_regs<32>(nv, A, w + L.grad, w + L.Mgrad);
-  KSYNC();
-  return bad ? ST_NOT_PD : 0;
-#else
+KDEV int newton_direction(const DModel& m, const Layout& L, float* w, int nefc, bool refactor, int nch,
+                          const unsigned long long* chmask, KProfAcc* pa) {
   int st = 0;
-  if (refactor) st = newton_factor<TRI_CACHE>(m, L, w, nefc, pa);
+#if WAVE == 64 && !MJK_BIG
+  if (TRI_CACHE && m.cone != 0) {
+    int nv = m.nv, nrow = cone_virtual_rows(m, L, w, nefc);
+    if (nrow >= 0) {
+      float* A = w + L.H;
+      hessian_tiles(nv, nrow, w + L.efc_J, w + L.efc_Dact, w + L.qM, [&](int i, int j, float v) {
+        A[i * nv + j] = v;
+        A[j * nv + i] = v;
+      });
+      KSYNC();
+      KPROF_MARK(pa, KP_SPARE);
+      int bad = nv <= 20 ? ldl_solve_regs<20>(nv, A, w + L.grad, w + L.Mgrad) : ldl_solve_regs<32>(nv, A, w + L.grad, w + L.Mgrad);
+      KSYNC();
+      return bad ? ST_NOT_PD : 0;
+    }
+    // the row buffer does not hold the cones' virtual rows
+    refactor = true;
+  }
+#endif
+  if (refactor || (nch && !(nch <= 2 && (!MJK_BIG || L.jw == 0) && newton_update(m, L, w, chmask))))
+    st = newton_factor<TRI_CACHE>(m, L, w, nefc, pa);
   KPROF_MARK(pa, KP_DIR);
   newton_solve(m, L, w);
   return st;
-#endif
 }
 
 // d1n: sum of the magnitudes of the slope's terms, the scale of its FP32
@@ -3618,29 +3729,18 @@ KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KP
   float *go = w + L.grad_old, *mgo = w + L.Mgrad_old, *Jaref = w + L.efc_Jaref;
   const float* Jv = w + L.efc_Jv;
   KPROF_MARK(pa, KP_SOLVE_INIT);
+  if (newton) {
+    st |= newton_direction<TRI_CACHE>(m, L, w, nefc, true, 0, nullptr, pa);
+    KPROF_MARK(pa, KP_NSOLVE);
+  } else {
+    for (int i = LANE; i < nv; i += WAVE) Mg[i] = grad[i];
+    KSYNC();
+    solve_ld(m, w + L.qLD, Mg);
+  }
+  for (int i = LANE; i < nv; i += WAVE) srch[i] = -Mg[i];
+  KSYNC();
   int it;
   for (it = 0; it < m.iterations; it++) {
-    if (newton) {
-      // H depends on qacc only through the active set: refactor only when it changed
-      st |= newton_direction<TRI_CACHE>(kfresh(m), kfresh(L), w, nefc, it == 0 || nch != 0, pa);
-      KPROF_MARK(pa, KP_NSOLVE);
-      for (int i = LANE; i < nv; i += WAVE) srch[i] = -Mg[i];
-    } else {
-      for (int i = LANE; i < nv; i += WAVE) Mg[i] = grad[i];
-      KSYNC();
-      solve_ld(m, w + L.qLD, Mg);
-      if (it == 0) {
-        for (int i = LANE; i < nv; i += WAVE) srch[i] = -Mg[i];
-      } else {
-        float nump = 0.f, denp = 0.f;
-        for (int i = LANE; i < nv; i += WAVE) { nump += grad[i] * (Mg[i] - mgo[i]); denp += go[i] * mgo[i]; }
-        float num = wsum(nump), den = wsum(denp);
-        float beta = num / fmaxf(KMINVAL, den);
-        if (beta < 0.f) beta = 0.f;
-        for (int i = LANE; i < nv; i += WAVE) srch[i] = -Mg[i] + beta * srch[i];
-      }
-    }
-    KSYNC();
     int exact = 0;
     KPROF_MARK(pa, KP_DIR);
     float dec = 0.f;
@@ -3659,7 +3759,8 @@ KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KP
     KSYNC();
     float oldcost = cost;
     KPROF_MARK(pa, KP_SOLVE_REST);
-    cost = cost_grad(kfresh(m), kfresh(L), w, nefc, &nch);
+    unsigned long long chm[2];
+    cost = cost_grad(kfresh(m), kfresh(L), w, nefc, &nch, true, chm);
     KPROF_MARK(pa, KP_COSTGRAD);
     float gp = 0.f;
     for (int i = LANE; i < nv; i += WAVE) gp += grad[i] * grad[i];
@@ -3670,6 +3771,25 @@ KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KP
     // a Newton step that stayed inside one quadratic piece (no row changed
     // zone) landed on that piece's stationary point: the exact minimiser
     if (newton && exact) break;
+    if (newton) {
+      // H depends on qacc only through the active set. (One call for both this
+      // direction and the first one, at the loop's head, costs the stored
+      // factor's kernels: 16384 quadrupeds 3.07 -> 3.19 ms, 64 399 -> 413 us.)
+      st |= newton_direction<TRI_CACHE>(kfresh(m), kfresh(L), w, nefc, false, nch, chm, pa);
+      KPROF_MARK(pa, KP_NSOLVE);
+      for (int i = LANE; i < nv; i += WAVE) srch[i] = -Mg[i];
+    } else {
+      for (int i = LANE; i < nv; i += WAVE) Mg[i] = grad[i];
+      KSYNC();
+      solve_ld(m, w + L.qLD, Mg);
+      float nump = 0.f, denp = 0.f;
+      for (int i = LANE; i < nv; i += WAVE) { nump += grad[i] * (Mg[i] - mgo[i]); denp += go[i] * mgo[i]; }
+      float num = wsum(nump), den = wsum(denp);
+      float beta = num / fmaxf(KMINVAL, den);
+      if (beta < 0.f) beta = 0.f;
+      for (int i = LANE; i < nv; i += WAVE) srch[i] = -Mg[i] + beta * srch[i];
+    }
+    KSYNC();
   }
   KPROF_MARK(pa, KP_DIR);
   // qfrc_constraint = J^T force at the final point, which the last
@@ -3719,7 +3839,7 @@ KDEV int st_integrate(const DModel& m, const Layout& L, float* w) {
     const float *qfs = w + L.qfrc_smooth, *qfc = w + L.qfrc_constraint;
     for (int k = LANE; k < nv; k += WAVE) acc[k] = qfs[k] + qfc[k];
     KSYNC();
-    if (solve_in_regs(m)) {
+    if (solve_in_regs<DENSE>(m)) {
       st |= smooth_solve_regs(nv, Bm, acc);
     } else {
       st |= factor_ld<DENSE>(m, Bm, A);
@@ -4117,11 +4237,30 @@ KDEV void run_env(const DModel& m, const Layout& L, float* w, const StepIO& io, 
   if (L.rand >= 0)
     for (int i = LANE; i < io.nrand; i += WAVE) w[L.rand + i] = io.rand[(size_t)env * io.nrand + i];
   KSYNC();
+  if (nsub == 0) {
+    // derived quantities of the current state only (no solve, no integration);
+    // apart from the loop below, whose registers its outputs would take (16384
+    // quadrupeds 3.07 -> 3.15 ms per control step as one pass of the loop)
+    st_kinematics(m, L, w);
+    st_com_pos(m, L, w);
+    st_crb(m, L, w);
+    if (nv > 0) factor_ld<(NPSET & 8) == 0>(m, w + L.qM, w + L.qLD);
+    st_com_vel(m, L, w);
+    st_smooth<(NPSET & 8) == 0>(m, L, w);
+    // the kinematics and dynamics intermediates are intact only here: the
+    // constraint rows of a full substep take their space
+    dump_ws(L, w, io.dump1, env);
+    if (io.has_aux) {
+      write_aux(m, L, w, io.aux, env);
+      write_cfrc_ext(m, L, w, io.aux, env, false);
+    }
+    return;
+  }
   int st = 0, niter = 0;
   KProfAcc pa;
   for (int i = 0; i < KP_N; i++) pa.t[i] = 0;
   KPROF_START(&pa);
-  for (int s = 0; s == 0 || s < nsub; s++) {
+  for (int s = 0; s < nsub; s++) {
     bool last = s == nsub - 1;
     st_kinematics(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_KIN);
@@ -4129,23 +4268,12 @@ KDEV void run_env(const DModel& m, const Layout& L, float* w, const StepIO& io, 
     KPROF_MARK(&pa, KP_COMPOS);
     st_crb(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_CRB);
-    if (nv > 0 && !solve_in_regs(m)) st |= factor_ld<(NPSET & 8) == 0>(kfresh(m), w + L.qM, w + L.qLD);
+    if (nv > 0 && !solve_in_regs<(NPSET & 8) == 0>(m)) st |= factor_ld<(NPSET & 8) == 0>(kfresh(m), w + L.qM, w + L.qLD);
     KPROF_MARK(&pa, KP_FACTOR);
     st_com_vel(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_COMVEL);
-    st |= st_smooth(kfresh(m), kfresh(L), w);
+    st |= st_smooth<(NPSET & 8) == 0>(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_SMOOTH);
-    if (nsub == 0) {
-      // derived quantities of the current state only (no solve, no
-      // integration); the kinematics and dynamics intermediates are intact only
-      // here: the constraint rows of a full substep take their space
-      dump_ws(L, w, io.dump1, env);
-      if (io.has_aux) {
-        write_aux(m, L, w, io.aux, env);
-        write_cfrc_ext(m, L, w, io.aux, env, false);
-      }
-      return;
-    }
     if (last && io.has_aux) write_aux(m, L, w, io.aux, env);
     if constexpr ((NPSET & 4) != 0)
       if (io.sensordata) st_sensors(kfresh(m), kfresh(L), w, io, env, s == 0, last);
