@@ -3345,7 +3345,8 @@ struct LsRows { float jar[2], jv[2], d[2]; int ty[2]; int on; const LsRow4* stag
 // point and, for the zone alone, at the reference) bound the humanoid's line
 // search by LDS latency: 16384 / 517 humanoids 6.17 -> 5.39 / 1.13 -> 0.90 ms
 // per control step. Not in the 168-VGPR kernels, whose registers they would
-// spill (16384 quadrupeds +2 %).
+// spill: kept for the search 16384 quadrupeds +2 %, read into an LsCone by every
+// evaluation +1.1 % (3.07 -> 3.10 ms), though quadrupeds have no such contact.
 struct LsCone { float x[6], v[6], D[6], f[5]; int dim; };
 
 KDEV void ls_cone(const DModel& m, const Layout& L, const float* w, int nefc, int q, LsCone* c) {
@@ -3462,7 +3463,8 @@ KDEV void ls_row(const DModel& m, const Layout& L, const float* w, int r, int ty
 
 // cost along search at alpha; nchange counts rows whose zone differs from
 // their zone at ref_alpha (0 means one quadratic piece spans both points)
-// KEEP: cone holds the lane's first elliptic contact
+// KEEP: cone holds the lane's first elliptic contact; else every evaluation
+// reads the contacts' rows from the workspace
 template <bool KEEP>
 KDEV LsPt ls_eval(const DModel& m, const Layout& L, float* w, int nefc, float alpha, float ref_alpha, const float* gq,
                   const LsRows& c, const LsCone& cone) {
@@ -3472,13 +3474,26 @@ KDEV LsPt ls_eval(const DModel& m, const Layout& L, float* w, int nefc, float al
     // elliptic contacts; the middle zone is not quadratic, so it never counts as one exact piece
     int ncon = iptr(w, L.misc)[MISC_NCON];
     for (int q = LANE; q < ncon; q += WAVE) {
-      LsCone o;
-      if (KEEP && q == LANE) o = cone;
-      else ls_cone(m, L, w, nefc, q, &o);
-      if (o.dim == 0) continue;
-      float cv, g1, g2, xr[6], Tr;
-      int z = ls_cone_line(o, alpha, &cv, &g1, &g2);
-      nch += z == 2 || z != ls_cone_zone(o, ref_alpha, xr, &Tr);
+      float cv, g1, g2;
+      int z, zr;
+      if constexpr (KEEP) {
+        LsCone o;
+        float xr[6], Tr;
+        if (q == LANE) o = cone;
+        else ls_cone(m, L, w, nefc, q, &o);
+        if (o.dim == 0) continue;
+        z = ls_cone_line(o, alpha, &cv, &g1, &g2);
+        zr = ls_cone_zone(o, ref_alpha, xr, &Tr);
+      } else {
+        const float* cr = w + L.con + CON_STRIDE * q;
+        int dim = iptr(cr, CON_NROW)[0], r0 = iptr(cr, CON_ROW0)[0];
+        if (dim < 2 || r0 + dim > nefc) continue;
+        const float *f5 = m.pair_friction + 5 * iptr(cr, CON_PAIR)[0], *x = w + L.efc_Jaref + r0, *v = w + L.efc_Jv + r0;
+        float sc = fric_scale(m, L, w), cr_, h1, h2;
+        z = k_ellip_line(x, v, w + L.efc_D + r0, f5, sc, dim, alpha, &cv, &g1, &g2);
+        zr = k_ellip_line(x, v, w + L.efc_D + r0, f5, sc, dim, ref_alpha, &cr_, &h1, &h2);
+      }
+      nch += z == 2 || z != zr;
       f += cv; d1 += g1; d2 += g2; d1a += fabsf(g1);
     }
   }
