@@ -794,7 +794,7 @@ KDEV int factor_ld(const DModel& m, const float* A, float* LD) {
 }
 
 #if WAVE == 64 && !MJK_BIG
-// x <- A^-1 x for a mass matrix A of nv <= NVM dofs (dense nv x nv), by MuJoCo's
+// x <- A^-1 x for a mass matrix A of at most 32 dofs (dense nv x nv), by MuJoCo's
 // L^T D L from the last dof to the first, with everything in registers: lane i
 // holds row i (column i, by symmetry) and x_i; step k broadcasts row k's leading
 // entries with readlane and the lanes before it take their multiples of them, x
@@ -803,15 +803,15 @@ KDEV int factor_ld(const DModel& m, const float* A, float* LD) {
 // level tables, LDS phases and separate register solve this replaces where the
 // factor is used once (qacc_smooth, the implicit velocity update). Eliminating
 // dof by dof rounds each entry once per descendant, the level sums once per
-// level: over 4000 humanoids (27 dofs) the RMS error of qacc_smooth against
-// FP64 is 1.30e-6 of its norm so, 1.12e-6 by levels and 0.87e-6 after one
-// refinement x += A^-1 (b - A x); over 4000 quadrupeds (18 dofs) 2.3e-7 both
-// ways. So the larger size refines (+0.04 ms of 0.81 at 517 humanoids), the
-// smaller doesn't need to. Bound by its instructions' issue, about two per pair
+// level, so one refinement x += A^-1 (b - A x) follows. RMS error of qacc_smooth
+// against the FP64 solution of the same FP32 system: 4000 humanoids (27 dofs)
+// 1.12e-6 of its norm by levels, 1.30e-6 so without the refinement, 0.87e-6
+// with it (+0.04 ms of 0.81 at 517 humanoids; with the error of the FP32 system
+// itself 2.01e-6 -> 1.90e-6); chains of 21 / 27 / 32 dofs half that of the levels. Bound by its instructions' issue, about two per pair
 // (k, j). Per control step: 16384 / 517 humanoids (implicit damping) 5.36 ->
-// 4.88 / 0.90 -> 0.84 ms. Elliptic cones only (solve_in_regs).
-template <int NVM>
-KDEV int ltdl_solve_regs(int nv, const float* A, float* x) {
+// 4.88 / 0.90 -> 0.84 ms. Where it runs: solve_in_regs.
+KDEV int smooth_solve_regs(int nv, const float* A, float* x) {
+  constexpr int NVM = SPARSE_ROWS_NV;
   float h[NVM];
   int ln = LANE < nv ? LANE : 0;
   kunroll<0, NVM>([&](auto j) { h[j] = j < nv ? A[j * nv + ln] : 0.f; });
@@ -829,7 +829,7 @@ KDEV int ltdl_solve_regs(int nv, const float* A, float* x) {
   });
   float id = 1.f / d, b = x[ln], r = b, v = 0.f;
 #pragma unroll 1
-  for (int pass = 0; pass < (NVM > 20 ? 2 : 1); pass++) {
+  for (int pass = 0; pass < 2; pass++) {
     if (pass) {
       kunroll<0, NVM>([&](auto j) {
         if (j < nv) r = fmaf(-A[j * nv + ln], rl_f(v, j), r);
@@ -858,14 +858,13 @@ KDEV int ltdl_solve_regs(int nv, const float* A, float* x) {
   KSYNC();
   return bad ? ST_M_NOT_PD : 0;
 }
-KDEV int smooth_solve_regs(int nv, const float* A, float* x) {
-  return nv <= 20 ? ltdl_solve_regs<20>(nv, A, x) : ltdl_solve_regs<32>(nv, A, x);
-}
-// Newton models with elliptic cones; the factor of qM itself is CG's
-// preconditioner, and pyramidal models keep the rounding of the level sums
-// (newton_direction says why). REGS: not the 168-VGPR kernels.
+// Newton models of 21 to 32 dofs with elliptic cones; the factor of qM itself is
+// CG's preconditioner, and pyramidal models keep the rounding of the level sums
+// (newton_direction says why). Smaller models keep the levels: unrefined, the
+// register solve had 1.12 (12 dofs) to 1.23 times (20) their error. REGS: not
+// the 168-VGPR kernels.
 template <bool REGS>
-KDEV bool solve_in_regs(const DModel& m) { return REGS && m.solver == 2 && m.cone != 0; }
+KDEV bool solve_in_regs(const DModel& m) { return REGS && m.solver == 2 && m.cone != 0 && m.nv > 20; }
 #else
 KDEV int smooth_solve_regs(int, const float*, float*) { return 0; }
 template <bool REGS>
