@@ -78,11 +78,11 @@ MJMLX_API int mjmlx_batched_capacity(const MjmlxBatchedSim* sim, int* maxcon, in
  * models of at most 32 dofs whose two workspaces fit a workgroup's LDS, two
  * more with 32 lanes per env (two envs per wave) at 256 registers and at 168
  * VGPRs, and, where the batch of a larger model has them, small LDS workspaces
- * first with a full-size rerun of the envs that need it (reported as 0); best of
- * two rounds after a warm-up round; keeps the fastest (choice:
+ * first with a full-size rerun of the envs that need it; best of two rounds
+ * after a warm-up round; keeps the fastest (choice:
  * 0 LDS, 1 device memory, 2 LDS at 168 VGPRs, 3 LDS at 512 registers,
  * 4 device memory at 168 VGPRs, 5 LDS with 32 lanes per env, 6 the same at
- * 168 VGPRs) and restores every buffer the timed steps wrote
+ * 168 VGPRs, 7 small LDS workspaces and a full-size rerun) and restores every buffer the timed steps wrote
  * (qpos, qvel, warm start, ctrl, solver statistics, sensor values and the
  * accelerometers' history, the aux outputs read by the get_xpos / cvel /
  * cfrc_ext getters), so the sim continues exactly as without the call; the
@@ -90,11 +90,16 @@ MJMLX_API int mjmlx_batched_capacity(const MjmlxBatchedSim* sim, int* maxcon, in
  * reference's kernels have one workspace placement per size class. */
 MJMLX_API int mjmlx_batched_autotune(MjmlxBatchedSim* sim, int steps, int* choice);
 
-/* Selects the step's kernel variant by the autotuner's numbering (0-6).
+/* The step's current kernel variant by the autotuner's numbering; 7 also where
+ * the sim was created so, its rerun then in LDS if the full workspace fits. */
+MJMLX_API int mjmlx_batched_variant(const MjmlxBatchedSim* sim);
+
+/* Selects the step's kernel variant by the autotuner's numbering (0-7).
  * Returns -1 for a variant the sim cannot run: an LDS variant when the
  * workspace exceeds a workgroup's LDS, a 32-lane variant for a model of more
- * than 32 dofs or whose two workspaces exceed it. A device-memory variant
- * allocates the workspaces on first selection. No reference counterpart. */
+ * than 32 dofs or whose two workspaces exceed it, 7 for a sim that was not
+ * created with small workspaces. A device-memory variant and 7 (its rerun)
+ * allocate the full workspaces in device memory on first selection. No reference counterpart. */
 MJMLX_API int mjmlx_batched_set_variant(MjmlxBatchedSim* sim, int choice);
 
 /* Learned warm start (mode 2): replay each control step's launches (features,

@@ -311,6 +311,10 @@ void place_big(MjmlxBatchedSim* s, const mjh::Caps& caps, const std::vector<mjh:
   s->high_occ = s->big_regs = false;
 }
 
+// the autotuner's number of small LDS workspaces with a full-size rerun
+// (try_compact); 0 .. VAR_N - 1 are the kernel variants
+enum { CHOICE_COMPACT = mjk::VAR_N };
+
 // kernel variant of the sim's current workspace placement and register budget
 int step_variant(const MjmlxBatchedSim* s) {
   if (s->use_gws) return s->high_occ ? mjk::VAR_GWS_OCC : mjk::VAR_GWS;
@@ -1269,13 +1273,13 @@ MJMLX_API int mjmlx_batched_autotune(MjmlxBatchedSim* s, int steps, int* choice)
       // at 512 registers (one wave per SIMD), 4 device memory at 168 VGPRs,
       // and for models that fit them, 32 lanes per env: 5 at 256 registers, 6
       // at 168 VGPRs
-      // and 7: small LDS workspaces first (try_compact), where the sim has them
-      const int ncand = can_compact ? 8 : (s->half_ok ? 7 : 5);
-      float ms[8];
-      std::fill(ms, ms + 8, 3.0e38f);
+      // and CHOICE_COMPACT: small LDS workspaces first, where the sim has them
+      const int ncand = can_compact ? CHOICE_COMPACT + 1 : (s->half_ok ? 7 : 5);
+      float ms[CHOICE_COMPACT + 1];
+      std::fill(ms, ms + CHOICE_COMPACT + 1, 3.0e38f);
       auto pick = [&](int g) {
-        s->compact = g == 7;
-        s->use_gws = g == 1 || g == 4 || g == 7;
+        s->compact = g == CHOICE_COMPACT;
+        s->use_gws = g == 1 || g == 4 || g == CHOICE_COMPACT;
         s->high_occ = g == 2 || g == 4 || g == 6;
         s->big_regs = g == 3;
         s->half = g == 5 || g == 6;
@@ -1308,14 +1312,21 @@ MJMLX_API int mjmlx_batched_autotune(MjmlxBatchedSim* s, int steps, int* choice)
       for (void* p : saved) HIPOK(hipFree(p));
       if (!s->use_gws && !had_gws) { HIPOK(hipFree(s->d_gws)); s->d_gws = nullptr; }
     }
-    if (choice) *choice = s->compact ? (int)mjk::VAR_LDS : step_variant(s);
+    if (choice) *choice = mjmlx_batched_variant(s);
     return 0;
   } catch (const std::exception& e) { report("mjmlx_batched_autotune", e); return -1; }
 }
 
+MJMLX_API int mjmlx_batched_variant(const MjmlxBatchedSim* s) {
+  if (!s) return -1;
+  return s->compact ? CHOICE_COMPACT : step_variant(s);
+}
+
 MJMLX_API int mjmlx_batched_set_variant(MjmlxBatchedSim* s, int choice) {
-  if (!s || choice < 0 || choice >= mjk::VAR_N) return -1;
-  bool gws = choice == 1 || choice == 4, half = choice == 5 || choice == 6;
+  if (!s || choice < 0 || choice > CHOICE_COMPACT) return -1;
+  if (choice == CHOICE_COMPACT && !s->d_kpc) return -1;
+  // the full-size rerun takes device memory, as when the autotuner times it
+  bool gws = choice == 1 || choice == 4 || choice == CHOICE_COMPACT, half = choice == 5 || choice == 6;
   if (!gws && !s->lds_ok) return -1;  // LDS variants: the workspace must fit a workgroup's LDS
   if (half && !s->half_ok) return -1;
   try {
@@ -1324,7 +1335,7 @@ MJMLX_API int mjmlx_batched_set_variant(MjmlxBatchedSim* s, int choice) {
     s->high_occ = choice == 2 || choice == 4 || choice == 6;
     s->big_regs = choice == 3;
     s->half = half;
-    s->compact = false;  // the chosen variant alone
+    s->compact = choice == CHOICE_COMPACT;
     return 0;
   } catch (const std::exception& e) { report("mjmlx_batched_set_variant", e); return -1; }
 }

@@ -97,6 +97,7 @@ def lib() -> C.CDLL:
             "mjmlx_batched_last_step_ms": (C.c_float, [C.c_void_p]),
             "mjmlx_batched_capacity": (C.c_int, [C.c_void_p, _I, _I, _I]),
             "mjmlx_batched_autotune": (C.c_int, [C.c_void_p, C.c_int, _I]),
+            "mjmlx_batched_variant": (C.c_int, [C.c_void_p]),
             "mjmlx_batched_set_variant": (C.c_int, [C.c_void_p, C.c_int]),
             "mjmlx_batched_set_graph": (C.c_int, [C.c_void_p, C.c_int]),
             "mjmlx_batched_debug_step": (C.c_int, [C.c_void_p, _F, _F, _F]),
@@ -294,11 +295,16 @@ class BatchedSim:
         """Time the step's kernel variants from the current state and keep the
         fastest; returns 0 (LDS workspace, 256 registers), 1 (device memory),
         2 (LDS workspace, 168 VGPRs), 3 (LDS workspace, 512 registers),
-        4 (device memory, 168 VGPRs), 5 (LDS workspace, 32 lanes per env) or
-        6 (the same at 168 VGPRs). The state is restored."""
+        4 (device memory, 168 VGPRs), 5 (LDS workspace, 32 lanes per env),
+        6 (the same at 168 VGPRs) or 7 (small LDS workspaces, full-size rerun of
+        the envs that need it). The state is restored."""
         c = C.c_int()
         assert lib().mjmlx_batched_autotune(self.h, steps, C.byref(c)) == 0
         return c.value
+
+    def variant(self) -> int:
+        """The current kernel variant by the autotuner's numbering."""
+        return lib().mjmlx_batched_variant(self.h)
 
     def set_variant(self, choice: int) -> bool:
         """Select the kernel variant by the autotuner's numbering; False when
