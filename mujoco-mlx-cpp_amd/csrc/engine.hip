@@ -261,27 +261,18 @@ void upload_kparams(MjmlxBatchedSim* s) {
 // 250 envs: 2.30 against 3.22 ms per control step), two take longer, so it is
 // used only where one round holds the batch. 8 boxes, 1000 envs: 4.9 -> 1.35 ms.
 // Results do not depend on which launch stepped an env.
-// A batch that neither size holds in one round goes to device memory: two LDS
-// rounds already take longer (9 boxes, 700 envs: 4.33 ms in three rounds, 2.32
-// from device memory; 6 boxes, 1100 envs: 3.70 against 2.07).
-// try_compact: true when the placement needs no change or small workspaces were set up.
+// try_compact: whether small workspaces were set up.
 bool try_compact(MjmlxBatchedSim* s, const mjh::Caps& caps, const std::vector<mjh::CollisionPair>& pairs,
-                 size_t lds_cu, size_t lds_max) {
+                 size_t lds_cu, size_t lds_max, size_t per_cu) {
   const auto& m = s->model;
-  // explicit capacities and placements are kept as given
-  for (const char* v : {"MJMLX_HIP_MAXCON", "MJMLX_HIP_MAXEFC", "MJMLX_HIP_LDS_MAX", "MJMLX_HIP_GLOBAL_WORKSPACE",
-                        "MJMLX_HIP_HIGH_OCC", "MJMLX_HIP_BIG_REGS", "MJMLX_HIP_REF_CAPS", "MJMLX_MAX_EFC"})
-    if (std::getenv(v)) return true;
-  size_t per_cu = ((size_t)s->B + s->ncu - 1) / std::max(1, s->ncu);
-  if (!s->use_gws && lds_cu / s->lds_bytes >= per_cu) return true;  // one round already
   // the accelerometers' history is written every substep: an env cannot be stepped twice
   if (m.nsensor > 0 || s->blob.proto.jw <= 0 || per_cu > 8) return false;
   size_t budget = std::min({lds_cu / per_cu / 1280 * 1280, lds_max});  // LDS is given out in 1280-byte pieces
-  int rpc = 1, fixed = 0, nfree = 0;
+  int rpc = 1, fixed = 0;
   for (auto& p : pairs)
     rpc = std::max(rpc, p.condim == 1 ? 1 : (m.cone == mjh::CONE_PYRAMIDAL ? 2 * (p.condim - 1) : p.condim));
   for (int k = 0; k < m.nv; k++) fixed += m.dof_frictionloss[k] > 0;
-  for (int j = 0; j < m.njnt; j++) fixed += (m.jnt_limited[j] ? 2 : 0), nfree += m.jnt_type[j] == mjk::JFREE;
+  for (int j = 0; j < m.njnt; j++) fixed += m.jnt_limited[j] ? 2 : 0;
   auto layout = [&](int c) {
     mjk::Layout l = mjk::make_layout(m.nq, m.nv, m.nu, m.nbody, m.njnt, m.ngeom, c, std::min(caps.maxefc, fixed + rpc * c),
                                      m.solver == mjh::SOL_NEWTON, s->nrand, s->blob.proto.jw, s->blob.proto.nM);
@@ -289,7 +280,7 @@ bool try_compact(MjmlxBatchedSim* s, const mjh::Caps& caps, const std::vector<mj
     l.con_cap = caps.con_cap;
     return l;
   };
-  int lo = std::min(caps.maxcon, std::max(16, 5 * nfree)), hi = caps.maxcon;
+  int lo = std::min(caps.maxcon, std::max(16, 5 * s->nfree)), hi = caps.maxcon;
   if (layout(lo).total * sizeof(float) > budget) return false;
   while (lo < hi) {
     int c = (lo + hi + 1) / 2;
@@ -304,9 +295,45 @@ bool try_compact(MjmlxBatchedSim* s, const mjh::Caps& caps, const std::vector<mj
   s->compact_variant = lds_cu / (s->Lc.total * sizeof(float)) <= 4 ? mjk::VAR_LDS_BIG : mjk::VAR_LDS;
   return true;
 }
+// Placement of a model of more than SPARSE_ROWS_NV dofs whose batch is not one
+// LDS round; `fits`: each env's full workspace alone fits LDS. ms per control
+// step, LDS rounds at full size / small workspaces / device memory:
+//   free bodies (6-9 boxes, CG and Newton, 600-4096 envs; landing): 6 boxes, 600
+//   envs 1.95 / 1.13 / 1.50; 8, 600 2.93 / 1.09 / 1.47; 8, 4096 15.7 / - / 3.8;
+//   Newton 6, 1100 2.42 / 1.17 / 1.73; 8, 2100 15.2 / - / 6.4. Small workspaces,
+//   else device memory, which two LDS rounds never beat.
+//   articulated, pyramidal cones, Newton or CG: small workspaces win (two
+//   quadrupeds, 36 dofs, 1100 envs 0.99 / 0.61 / 0.97, standing 1.93 / 1.70 /
+//   2.56; a 54-dof tree, 300 envs 2.90 / 1.73 / 2.54). Device memory holds 8
+//   envs per CU and is up to 1.55 times slower a round: with three LDS rounds to
+//   one or two standing quadrupeds lose (three of them, 1100 envs 4.38 / - / 5.16;
+//   two, 2100 envs 2.73 / - / 3.07; a 40-dof chain, 2100 envs 3.31 / - / 3.80),
+//   from four times its rounds all gain (three quadrupeds, 4096 envs 6.2 / - /
+//   4.5; the tree, 1100 envs 10.6 / - / 5.9; a 66-dof scene 8.0 / - / 7.4).
+//   articulated with elliptic cones under Newton: H is factored in the workspace
+//   at every step; no batch of them was measured to gain. They stay in LDS.
+// A workspace set in device memory that cannot be allocated goes back to LDS.
 void place_big(MjmlxBatchedSim* s, const mjh::Caps& caps, const std::vector<mjh::CollisionPair>& pairs, size_t lds_cu,
                size_t lds_max) {
-  if (s->nv <= mjk::SPARSE_ROWS_NV || try_compact(s, caps, pairs, lds_cu, lds_max)) return;
+  const auto& m = s->model;
+  if (s->nv <= mjk::SPARSE_ROWS_NV) return;
+  // explicit capacities, row forms and placements are kept as given
+  for (const char* v : {"MJMLX_HIP_MAXCON", "MJMLX_HIP_MAXEFC", "MJMLX_HIP_LDS_MAX", "MJMLX_HIP_GLOBAL_WORKSPACE",
+                        "MJMLX_HIP_HIGH_OCC", "MJMLX_HIP_BIG_REGS", "MJMLX_HIP_REF_CAPS", "MJMLX_MAX_EFC",
+                        "MJMLX_HIP_DENSE_ROWS"})
+    if (std::getenv(v)) return;
+  size_t per_cu = ((size_t)s->B + s->ncu - 1) / std::max(1, s->ncu);
+  bool fits = !s->use_gws, free_bodies = 6 * s->nfree == s->nv;
+  if (fits && lds_cu / s->lds_bytes >= per_cu) return;  // one round already
+  if (!free_bodies && m.solver == mjh::SOL_NEWTON && m.cone != mjh::CONE_PYRAMIDAL) return;
+  if (try_compact(s, caps, pairs, lds_cu, lds_max, per_cu) || !fits) return;
+  size_t in_lds = lds_cu / s->lds_bytes, lds_rounds = (per_cu + in_lds - 1) / in_lds;
+  if (!free_bodies && lds_rounds < 4 * ((per_cu + 7) / 8)) return;
+  if (hipMalloc(&s->d_gws, (size_t)s->B * s->L.total * sizeof(float)) != hipSuccess) {
+    (void)hipGetLastError();
+    s->d_gws = nullptr;
+    return;
+  }
   s->use_gws = true;
   s->high_occ = s->big_regs = false;
 }
@@ -759,7 +786,7 @@ MJMLX_API MjmlxBatchedSim* mjmlx_batched_create(const MjmlxModel* model, const M
       if (const char* v = std::getenv("MJMLX_HIP_HIGH_OCC")) s->high_occ = std::atoi(v) != 0;
     }
     place_big(s, caps, pairs, lds_cu, lds_max);
-    if (s->use_gws) HIPOK(hipMalloc(&s->d_gws, (size_t)s->B * s->L.total * sizeof(float)));
+    if (s->use_gws && !s->d_gws) HIPOK(hipMalloc(&s->d_gws, (size_t)s->B * s->L.total * sizeof(float)));
     HIPOK(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
     HIPOK(hipEventCreate(&s->ev0));
     HIPOK(hipEventCreate(&s->ev1));

@@ -2,10 +2,13 @@
 and what selects it again."""
 from __future__ import annotations
 
+import re
+
 import numpy as np
 import pytest
 
 from mjmlx_hip import capi, scenes
+from test_reference_models import model_xml
 from test_gpu_compact import _states
 
 pytestmark = pytest.mark.gpu
@@ -43,3 +46,46 @@ def test_refused_where_the_sim_has_none():
         sim = capi.BatchedSim(model, B)
         v = sim.variant()
         assert v != COMPACT and not sim.set_variant(COMPACT) and sim.variant() == v
+
+
+def _side_by_side(xml, n):
+    """n copies of a scene's bodies and actuators, 3 m apart."""
+    xml = re.sub(r"<contact>.*?</contact>", "", xml, flags=re.S)  # excludes name the bodies
+    a, b = xml.index("<body"), xml.index("</worldbody>")
+    c, d = xml.index("<actuator>") + len("<actuator>"), xml.index("</actuator>")
+    name = lambda t, k: re.sub(r'\b(name|joint|site)="([^"]+)"', rf'\1="\2_{k}"', t)  # noqa: E731
+    x = re.compile(r'(<body[^>]*? pos=")([-\d.]+)')
+    bodies = "".join(x.sub(lambda m: f"{m[1]}{float(m[2]) + 3 * k}", name(xml[a:b], k), count=1) for k in range(n))  # noqa: B023
+    return xml[:a] + bodies + xml[b:c] + "".join(name(xml[c:d], k) for k in range(n)) + xml[d:]
+
+
+def _model(name):
+    if name == "tree54":
+        return model_xml("high_dof_tree")
+    kind, n = name[:-1], int(name[-1])
+    if kind == "boxes":
+        return scenes.boxes_xml(n, 100 + n)
+    if kind == "quadrupeds":
+        return _side_by_side(scenes.quadruped_xml(self_collision=False), n)
+    return _side_by_side(scenes.humanoid_xml(self_collision=False), n)
+
+
+LDS, DEVICE = 3, 1  # at most four envs of these per CU: the whole register file
+
+
+# A model of more than 32 dofs keeps LDS unless another placement was measured to
+# be faster for its kind: free bodies go to small workspaces or device memory,
+# articulated models to small workspaces, to device memory only from four times
+# its rounds on, and with elliptic cones under Newton they stay.
+@pytest.mark.parametrize("name,B,want", [
+    ("boxes6", 300, LDS), ("boxes6", 600, COMPACT), ("boxes6", 2100, DEVICE), ("boxes8", 4096, DEVICE),
+    ("quadrupeds2", 300, LDS), ("quadrupeds2", 1100, COMPACT), ("quadrupeds2", 2100, LDS), ("quadrupeds2", 4096, LDS),
+    ("quadrupeds3", 1100, LDS), ("quadrupeds3", 4096, DEVICE), ("tree54", 300, COMPACT), ("tree54", 1100, DEVICE),
+    ("humanoids2", 300, LDS), ("humanoids2", 1100, LDS)])
+def test_default_placement(name, B, want):
+    assert capi.BatchedSim(capi.Model(_model(name)), B).variant() == want
+
+
+def test_dense_rows_keep_the_given_placement(monkeypatch):
+    monkeypatch.setenv("MJMLX_HIP_DENSE_ROWS", "1")
+    assert capi.BatchedSim(capi.Model(scenes.boxes_xml(6, 106)), 2100).variant() == LDS
