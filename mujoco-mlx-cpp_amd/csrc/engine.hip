@@ -177,7 +177,7 @@ struct MjmlxBatchedSim {
   hipGraphExec_t gexec = nullptr;
   int g_n = -1, g_cur = -1, g_mode = -1;
   const void *g_mlp = nullptr, *g_xb = nullptr;
-  bool g_gws = false, g_occ = false, g_big = false, g_half = false;
+  bool g_gws = false, g_occ = false, g_big = false, g_half = false, g_compact = false;
   // packed readback
   int* d_pack_bodies = nullptr;
   float* d_pack = nullptr;
@@ -455,7 +455,7 @@ bool step_graph(MjmlxBatchedSim* s, int n) {
   s->mlp->ensure(s->B);  // allocations happen before any capture
   if (!s->gexec || s->g_n != n || s->g_cur != s->feat_cur || s->g_mlp != s->mlp || s->g_xb != s->mlp->xb ||
       s->g_mode != s->feat_mode || s->g_gws != s->use_gws || s->g_occ != s->high_occ || s->g_big != s->big_regs ||
-      s->g_half != s->half) {
+      s->g_half != s->half || s->g_compact != s->compact) {
     if (s->gexec) { HIPOK(hipGraphExecDestroy(s->gexec)); s->gexec = nullptr; }
     if (s->graph) { HIPOK(hipGraphDestroy(s->graph)); s->graph = nullptr; }
     HIPOK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
@@ -464,7 +464,7 @@ bool step_graph(MjmlxBatchedSim* s, int n) {
     HIPOK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
     s->g_n = n; s->g_cur = s->feat_cur; s->g_mlp = s->mlp; s->g_xb = s->mlp->xb;
     s->g_mode = s->feat_mode; s->g_gws = s->use_gws; s->g_occ = s->high_occ; s->g_big = s->big_regs;
-    s->g_half = s->half;
+    s->g_half = s->half; s->g_compact = s->compact;
   }
   HIPOK(hipEventRecord(s->ev0, s->stream));
   HIPOK(hipGraphLaunch(s->gexec, s->stream));
@@ -1467,6 +1467,8 @@ MJMLX_API int mjmlx_batched_set_warmstart_mlp(MjmlxBatchedSim* s, MjmlxMLP* mlp)
   }
   try {
     ensure_learned(s);
+    // a network may have the address of a freed one, and a captured step its buffers
+    s->g_mlp = nullptr;
     s->mlp = mlp;
     return 0;
   } catch (const std::exception& e) { report("mjmlx_batched_set_warmstart_mlp", e); return -1; }

@@ -89,3 +89,54 @@ def test_default_placement(name, B, want):
 def test_dense_rows_keep_the_given_placement(monkeypatch):
     monkeypatch.setenv("MJMLX_HIP_DENSE_ROWS", "1")
     assert capi.BatchedSim(capi.Model(scenes.boxes_xml(6, 106)), 2100).variant() == LDS
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_captured_step_follows_the_variant(graph):
+    """A learned control step captured as a graph is captured again when the
+    variant changes, also where only small workspaces go. Both variants give the
+    same bits, so the time tells: 8 boxes, 600 envs take about 2.5 times as long
+    in full-size LDS workspaces."""
+    n, B = 8, 600
+    model = capi.Model(scenes.boxes_xml(n, 108))
+    rng = np.random.default_rng(0)
+    sim = capi.BatchedSim(model, B)
+    assert sim.variant() == COMPACT
+    sim.set_state(_states(model, n, B, np.zeros(B, bool), rng), np.zeros((B, 6 * n), np.float32))
+    sim.set_warmstart_mlp(capi.MLP(sim.feature_dim(), 64, 6 * n, seed=1))
+    assert sim.set_warmstart_mode(2) == 0
+    sim.set_graph(graph)
+    ms = []
+    for v in (COMPACT, 3):
+        assert sim.variant() == v or sim.set_variant(v)
+        t = []
+        for _ in range(6):
+            sim.step(None, 2)
+            sim.sync()
+            t.append(sim.last_step_ms())
+        ms.append(float(np.median(t[2:])))
+    print(f"graph {graph}: small workspaces {ms[0]:.3f} ms, full-size LDS {ms[1]:.3f}")
+    assert ms[1] > 1.6 * ms[0]
+
+
+def test_captured_step_follows_the_network():
+    """A network freed and another made, which may get the first one's address."""
+    B = 64
+    model = capi.Model(scenes.quadruped_xml())
+    out = []
+    for graph in (False, True):
+        sim = capi.BatchedSim(model, B)
+        sim.set_graph(graph)
+        for seed, width in ((1, 64), (2, 128), (3, 64)):
+            net = capi.MLP(sim.feature_dim(), width, model.nv, seed=seed)
+            net.set_normalization(out_std=np.full(model.nv, 20.0))
+            sim.set_warmstart_mlp(net)
+            assert sim.set_warmstart_mode(2) == 0
+            for _ in range(4):
+                sim.step(None, 2)
+            out.append((*sim.state(), sim.stats()["niter"]))
+            sim.set_warmstart_mlp(None)
+            del net
+    for a, b in zip(out[:3], out[3:]):
+        for x, y in zip(a, b):
+            assert np.array_equal(x, y)
