@@ -122,7 +122,11 @@ MJMLX_API int mjmlx_batched_debug_step(MjmlxBatchedSim* sim, const float* ctrl, 
  * unsigned long long[num_envs * 17].
  * Returns -1 in the product build. */
 MJMLX_API int mjmlx_batched_profile_step(MjmlxBatchedSim* sim, const float* ctrl, int nsub, unsigned long long* out);
-/* offset / length (floats) / kind (0 float, 1 int) of a workspace field */
+/* offset / length (floats) / kind (0 float, 1 int) of a workspace field. qM and
+ * its factor qLD are nv x nv floats or, where the length is smaller, compact
+ * rows: a dof's diagonal, then its dof ancestors' entries, nearest first (beyond
+ * 64 dofs; from 33 where every dof tree is a path of at most 8 dofs, such as
+ * free bodies). */
 MJMLX_API int mjmlx_batched_layout(const MjmlxBatchedSim* sim, const char* name, int* off, int* len, int* kind);
 
 /* ---- learned warm start (no counterpart in the reference) ----------------

@@ -4258,7 +4258,7 @@ KDEV void run_env(const DModel& m, const Layout& L, float* w, const StepIO& io, 
     st_kinematics(m, L, w);
     st_com_pos(m, L, w);
     st_crb(m, L, w);
-    if (nv > 0) factor_ld<(NPSET & 8) == 0>(m, w + L.qM, w + L.qLD);
+    if (nv > 0 && (!solve_in_regs<(NPSET & 8) == 0>(m) || io.dump1)) factor_ld<(NPSET & 8) == 0>(m, w + L.qM, w + L.qLD);
     st_com_vel(m, L, w);
     st_smooth<(NPSET & 8) == 0>(m, L, w);
     // the kinematics and dynamics intermediates are intact only here: the
@@ -4282,7 +4282,8 @@ KDEV void run_env(const DModel& m, const Layout& L, float* w, const StepIO& io, 
     KPROF_MARK(&pa, KP_COMPOS);
     st_crb(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_CRB);
-    if (nv > 0 && !solve_in_regs<(NPSET & 8) == 0>(m)) st |= factor_ld<(NPSET & 8) == 0>(kfresh(m), w + L.qM, w + L.qLD);
+    // a dump shows qM's factor also where the solves do without it
+    if (nv > 0 && (!solve_in_regs<(NPSET & 8) == 0>(m) || (last && io.dump1))) st |= factor_ld<(NPSET & 8) == 0>(kfresh(m), w + L.qM, w + L.qLD);
     KPROF_MARK(&pa, KP_FACTOR);
     st_com_vel(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_COMVEL);

@@ -388,7 +388,25 @@ class DebugDump:
     def get(self, which: int, env: int, name: str) -> np.ndarray:
         off, ln, kind = self.sim.layout(name)
         seg = self.d[which][env * self.total + off: env * self.total + off + ln].copy()
+        nv = self.sim.nv
+        if name in ("qM", "qLD") and nv <= 64 and ln < nv * nv:
+            return self._dense(seg, which, env, name).ravel()
         return seg.view(np.int32) if kind == 1 else seg
+
+    def _dense(self, rows, which: int, env: int, name: str) -> np.ndarray:
+        """nv x nv from compact rows (a dof's diagonal, then its ancestors nearest
+        first); above the diagonal qM's entries, for its factor too."""
+        nv, parent = self.sim.nv, self.sim.model.field("dof_parentid").astype(int)
+        out = np.zeros((nv, nv), np.float32) if name == "qM" else self.get(which, env, "qM").reshape(nv, nv)
+        t = 0
+        for i in range(nv):
+            j = i
+            while j >= 0:
+                out[i, j] = rows[t]
+                if name == "qM":
+                    out[j, i] = rows[t]
+                t, j = t + 1, parent[j]
+        return out
 
 
 class MLP:
