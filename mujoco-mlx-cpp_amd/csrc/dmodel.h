@@ -113,9 +113,9 @@ struct DModel {
   //   dof   body, damping, stiffness (hinges and slides), 0 / qpos address, qpos_spring, first actuator, actuators
   //   geom  pos, body / quat
   //   act   actuator, qpos address, ctrllimited | forcelimited << 1, gear / gain[0], bias[0..2] / ctrlrange, forcerange
-  //   pair  geom1 | geom2 << 16, type1 | type2 << 8 | both bounded << 16, bounding radii + margin, margin
+  //   pair  geom1 | type1 << 24 | both bounded << 28, geom2 | type2 << 24, bounding radii + margin, margin
   const MJK_G int *body_rec, *jnt_rec, *dof_rec, *geom_rec, *act_rec, *pair_rec;
-  const MJK_G int* ment;  // qM's tree entries i | j << 16, dof by dof, from the dof up its chain
+  const MJK_G int* ment;  // qM's tree entries (i, j), dof by dof, from the dof up its chain
 };
 enum { BODY_REC = 24, JNT_REC = 8, DOF_REC = 8, GEOM_REC = 8, ACT_REC = 12, PAIR_REC = 4 };
 // sensor kinds (MuJoCo mjtSensor)

@@ -362,7 +362,7 @@ Blob build_blob(const Model& m, std::vector<CollisionPair>* pairs_out) {
     bool lin = m.jnt_type[j] == JNT_HINGE || m.jnt_type[j] == JNT_SLIDE;
     r[0] = m.dof_bodyid[k]; r[1] = fb(m.dof_damping[k]); r[2] = lin ? fb(m.jnt_stiffness[j]) : 0;
     r[4] = qa; r[5] = lin ? fb(m.qpos_spring[qa]) : 0; r[6] = dof_act_adr[k]; r[7] = dof_act_num[k];
-    for (int a = 0; a < nchain[k]; a++) ment.push_back(k | chain[(size_t)k * MAX_DOF_DEPTH + a] << 16);
+    for (int a = 0; a < nchain[k]; a++) { ment.push_back(k); ment.push_back(chain[(size_t)k * MAX_DOF_DEPTH + a]); }
   }
   for (int g = 0; g < m.ngeom; g++) {
     int* r = &geom_rec[(size_t)g * GEOM_REC];
@@ -382,18 +382,18 @@ Blob build_blob(const Model& m, std::vector<CollisionPair>* pairs_out) {
   for (int i = 0; i < np; i++) {
     int* r = &pair_rec[(size_t)i * PAIR_REC];
     float r1 = (float)m.geom_rbound[pg1[i]], r2 = (float)m.geom_rbound[pg2[i]];
-    r[0] = pg1[i] | pg2[i] << 16;
-    r[1] = m.geom_type[pg1[i]] | m.geom_type[pg2[i]] << 8 | (r1 > 0.f && r2 > 0.f ? 0x10000 : 0);
+    r[0] = pg1[i] | m.geom_type[pg1[i]] << 24 | (r1 > 0.f && r2 > 0.f ? 1 << 28 : 0);
+    r[1] = pg2[i] | m.geom_type[pg2[i]] << 24;
     r[2] = __builtin_bit_cast(int, r1 + r2 + pmg[i]); r[3] = __builtin_bit_cast(int, pmg[i]);
   }
-  if (m.ngeom > 65535) throw std::runtime_error("HIP engine: more than 65535 geoms");
+  if (m.ngeom >= 1 << 24) throw std::runtime_error("HIP engine: 2^24 geoms or more");
 
   Blob blob;
   Builder B;
   DModel& d = blob.proto;
   std::memset(&d, 0, sizeof(d));
   d.nM = nM;
-  d.nment = (int)ment.size();
+  d.nment = (int)ment.size() / 2;
   d.ntree = (int)tree_adr.size() - 1;
   d.nq = m.nq; d.nv = nv; d.nu = m.nu; d.nbody = nb; d.njnt = m.njnt; d.ngeom = m.ngeom; d.npair = np;
   d.nlevel = maxd; d.ndoflevel = ndl; d.nflev = (int)flev_adr.size() - 1; d.nfloss = (int)floss_dof.size(); d.nlim = (int)lim_jnt.size();

@@ -641,7 +641,7 @@ KDEV void st_crb(const DModel& m, const Layout& L, float* w) {
   // one lane per tree entry (i, j), j on i's chain from i up (the order of the
   // compact rows)
   for (int t = LANE; t < m.nment; t += WAVE) {
-    int ij = m.ment[t], i = ij & 0xffff, j = ij >> 16;
+    int i = m.ment[2 * t], j = m.ment[2 * t + 1];
     const float *bi = buf + 6 * i, *cj = cdof + 6 * j;
     float s = cj[0] * bi[0] + cj[1] * bi[1] + cj[2] * bi[2] + cj[3] * bi[3] + cj[4] * bi[4] + cj[5] * bi[5];
     if (i == j) s += m.dof_armature[i];
@@ -1947,16 +1947,16 @@ KDEV int st_collision(const DModel& m, const Layout& L, float* w) {
     RawC rc[MAXC_PAIR];
     int cnt = 0;
     if (p < m.npair) {
-      ki4 pr = kld4(m.pair_rec + PAIR_REC * p);  // geoms, types and cull flag, reach (radii + margin), margin
-      int g1 = pr[0] & 0xffff, g2 = (int)((unsigned)pr[0] >> 16);
+      ki4 pr = kld4(m.pair_rec + PAIR_REC * p);  // geoms with types and the cull flag, reach (radii + margin), margin
+      int g1 = pr[0] & 0xffffff, g2 = pr[1] & 0xffffff;
       const float *x1 = gx + 3 * g1, *x2 = gx + 3 * g2;
       float margin = ki2f(pr[3]);
       bool cull = false;
-      if (pr[1] & 0x10000) {
+      if (pr[0] & (1 << 28)) {
         float dv[3] = {x1[0] - x2[0], x1[1] - x2[1], x1[2] - x2[2]};
         cull = sqrtf(dot3(dv, dv)) > ki2f(pr[2]);
       }
-      if (!cull) cnt = k_narrow<NPSET>(pr[1] & 0xff, (pr[1] >> 8) & 0xff, m.geom_size + 3 * g1, m.geom_size + 3 * g2,
+      if (!cull) cnt = k_narrow<NPSET>((pr[0] >> 24) & 15, pr[1] >> 24, m.geom_size + 3 * g1, m.geom_size + 3 * g2,
                                 x1, gm + 9 * g1, x2, gm + 9 * g2, margin, rc);
     }
     int badp = cnt < 0 ? 1 : 0;
