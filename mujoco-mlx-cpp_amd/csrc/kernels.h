@@ -608,14 +608,14 @@ KDEV void st_com_pos(const DModel& m, const Layout& L, float* w) {
 // dense nv x nv
 KDEV bool m_compact(const DModel& m) { return MJK_BIG && (m.nv > COMPACT_M_NV || (m.nv > SPARSE_ROWS_NV && m.ntree > 0)); }
 // index of entry (i, j), j == i or a dof ancestor of i (any j when dense)
-KDEV int mxi(const DModel& m, int i, int j) {
-  return m_compact(m) ? m.dof_madr[i] + m.dof_depth[i] - m.dof_depth[j] : i * m.nv + j;
+KDEV int mxi(const DModel& m, bool compact, int i, int j) {
+  return compact ? m.dof_madr[i] + m.dof_depth[i] - m.dof_depth[j] : i * m.nv + j;
 }
 
 // entry (i, j), j <= i, of qM in either storage (zero off the dof tree)
 KDEV float m_entry(const DModel& m, const float* M, int i, int j) {
   if (!m_compact(m)) return M[i * m.nv + j];
-  return i < m.dof_subtree_end[j] ? M[mxi(m, i, j)] : 0.f;  // j is i or an ancestor
+  return i < m.dof_subtree_end[j] ? M[mxi(m, true, i, j)] : 0.f;  // j is i or an ancestor
 }
 
 // mj_crb: composite inertia by subtree ranges, then qM entries along each dof's
@@ -758,7 +758,7 @@ KDEV int factor_ld(const DModel& m, const float* A, float* LD) {
           if (!(dk > KMINVAL)) { bad = 1; dk = KMINVAL; }
           acc += rk[d - m.dof_depth[i]] * rk[d - m.dof_depth[j]] / dk;
         }
-        LD[mxi(m, i, j)] -= acc;
+        LD[mxi(m, true, i, j)] -= acc;
       } else {
         for (int q = m.flev_kadr[e]; q < m.flev_kadr[e] + m.flev_kcnt[e]; q++) {
           int k = m.flev_k[q];
@@ -1037,22 +1037,27 @@ KDEV void solve_ld(const DModel& m, const float* LD, float* x) {
     solve_ld_trees(m, LD, x);
     return;
   }
+  // past the register solve every matrix on 64 lanes is compact. Left to
+  // m_compact the choice is a branch among the index loads of every entry, one
+  // more load to wait for (64 envs, 3 chains of 30 dofs: 2.94 ms per control step
+  // so, 2.32 without it; 10 chains of 12 dofs 0.81 and 0.72)
+  const bool compact = WAVE == 64 || m_compact(m);
   for (int lv = m.ndoflevel - 2; lv >= 0; lv--) {
     for (int t = m.doflevel_adr[lv] + LANE; t < m.doflevel_adr[lv + 1]; t += WAVE) {
       int i = m.doflevel_dof[t];
       float acc = 0.f;
-      for (int k = i + 1; k < m.dof_subtree_end[i]; k++) acc += LD[mxi(m, k, i)] * x[k];
+      for (int k = i + 1; k < m.dof_subtree_end[i]; k++) acc += LD[mxi(m, compact, k, i)] * x[k];
       x[i] -= acc;
     }
     KSYNC();
   }
-  for (int i = LANE; i < nv; i += WAVE) x[i] /= LD[mxi(m, i, i)];
+  for (int i = LANE; i < nv; i += WAVE) x[i] /= LD[mxi(m, compact, i, i)];
   KSYNC();
   for (int lv = 1; lv < m.ndoflevel; lv++) {
     for (int t = m.doflevel_adr[lv] + LANE; t < m.doflevel_adr[lv + 1]; t += WAVE) {
       int k = m.doflevel_dof[t];
       float acc = 0.f;
-      for (int i = m.dof_parentid[k]; i >= 0; i = m.dof_parentid[i]) acc += LD[mxi(m, k, i)] * x[i];
+      for (int i = m.dof_parentid[k]; i >= 0; i = m.dof_parentid[i]) acc += LD[mxi(m, compact, k, i)] * x[i];
       x[k] -= acc;
     }
     KSYNC();
@@ -2270,7 +2275,7 @@ KDEV float mulM_row(const DModel& m, const float* M, const float* x, int i) {
   const float* row = M + m.dof_madr[i];  // the diagonal, then the ancestors
   int a = 1;
   for (int j = m.dof_parentid[i]; j >= 0; j = m.dof_parentid[j], a++) acc += row[a] * x[j];
-  for (int k = i; k < m.dof_subtree_end[i]; k++) acc += M[mxi(m, k, i)] * x[k];
+  for (int k = i; k < m.dof_subtree_end[i]; k++) acc += M[mxi(m, true, k, i)] * x[k];
   return acc;
 }
 
@@ -3833,7 +3838,8 @@ KDEV int st_integrate(const DModel& m, const Layout& L, float* w) {
   if (implicit || damp) {
     float* A = w + L.qLD;  // scratch: qLD of M is dead after the solver
     float* Bm = w + L.qM;   // M + h*D built in place of qM (dead after the solver)
-    for (int k = LANE; k < nv; k += WAVE) Bm[mxi(m, k, k)] += h * m.dof_damping[k];
+    const bool compact = m_compact(m);
+    for (int k = LANE; k < nv; k += WAVE) Bm[mxi(m, compact, k, k)] += h * m.dof_damping[k];
     KSYNC();
     if (implicit) {
       const float* af = w + L.act_force;
@@ -3846,7 +3852,7 @@ KDEV int st_integrate(const DModel& m, const Layout& L, float* w) {
           if (m.act_forcelimited[u] && (f <= m.act_forcerange[2 * u] || f >= m.act_forcerange[2 * u + 1])) continue;
           add -= h * m.act_gear[u] * m.act_gear[u] * m.act_bias[3 * u + 2];
         }
-        Bm[mxi(m, k, k)] += add;
+        Bm[mxi(m, compact, k, k)] += add;
       }
       KSYNC();
     }
