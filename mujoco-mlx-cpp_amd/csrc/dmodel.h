@@ -74,7 +74,7 @@ struct DModel {
   float magnetic[3];
   // pointers only from here on: Blob::bind relocates every word from body_rootid on
   // bodies
-  const MJK_G int *body_rootid, *body_subtree_end, *body_lastdof;
+  const MJK_G int *body_rootid, *body_subtree_end, *body_lastdof, *level_adr;
   const MJK_G float *body_ipos, *body_iquat, *body_mass, *body_inertia,
       *body_subtreemass, *body_invweight0;
   // joints
@@ -114,10 +114,12 @@ struct DModel {
   //   geom  pos, body / quat
   //   act   actuator, qpos address, ctrllimited | forcelimited << 1, gear / gain[0], bias[0..2] / ctrlrange, forcerange
   //   pair  geom1 | type1 << 24 | both bounded << 28, geom2 | type2 << 24, bounding radii + margin, margin
-  const MJK_G int *body_rec, *jnt_rec, *dof_rec, *geom_rec, *act_rec, *pair_rec;
+  //   level body, parent, first joint, joints | dofs << 16 / dof address, joint types, 0, 0: of every
+  //         body but the world, level by level from level_adr
+  const MJK_G int *body_rec, *level_rec, *jnt_rec, *dof_rec, *geom_rec, *act_rec, *pair_rec;
   const MJK_G int* ment;  // qM's tree entries (i, j), dof by dof, from the dof up its chain
 };
-enum { BODY_REC = 24, JNT_REC = 8, DOF_REC = 8, GEOM_REC = 8, ACT_REC = 12, PAIR_REC = 4 };
+enum { BODY_REC = 24, LEVEL_REC = 8, JNT_REC = 8, DOF_REC = 8, GEOM_REC = 8, ACT_REC = 12, PAIR_REC = 4 };
 // sensor kinds (MuJoCo mjtSensor)
 enum { SENS_ACCELEROMETER = 1, SENS_VELOCIMETER = 2, SENS_GYRO = 3, SENS_MAGNETOMETER = 6, SENS_JOINTPOS = 9,
        SENS_JOINTVEL = 10, SENS_ACTUATORPOS = 13, SENS_ACTUATORVEL = 14, SENS_JOINTACTFRC = 16, SENS_BALLQUAT = 18,

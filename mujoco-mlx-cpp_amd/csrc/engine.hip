@@ -350,6 +350,10 @@ int step_variant(const MjmlxBatchedSim* s) {
   return s->big_regs ? mjk::VAR_LDS_BIG : mjk::VAR_LDS;
 }
 
+// whether the model needs the kernels for any size: more dofs than the small
+// ones take, or more bodies than lanes (LevelBodies)
+bool big_kernels(const MjmlxBatchedSim* s) { return s->nv > mjk::SPARSE_ROWS_NV || s->nb > 64; }
+
 // one workgroup (one wave) per env: the kernel variant for the workspace
 // placement (device memory, LDS at three, two or one waves per SIMD), compiled
 // for the model's narrow-phase set and, with sensors, the sensor stage
@@ -364,7 +368,7 @@ void launch_step(MjmlxBatchedSim* s, mjk::StepIO io, int nsub) {
   }
   mjk::StepLaunch l{s->d_kp, s->B, 0, step_variant(s), s->lds_bytes, s->d_gws, s->stream,
                     mjk::ls_cache_rows(s->L.maxefc)};
-  mjk::launch_step_np(s->npset | (s->model.nsensor > 0 ? 4 : 0), s->nv > mjk::SPARSE_ROWS_NV, l, io, nsub);
+  mjk::launch_step_np(s->npset | (s->model.nsensor > 0 ? 4 : 0), big_kernels(s), l, io, nsub);
 }
 
 mjk::StepIO make_io(MjmlxBatchedSim* s, float* dump1, float* dump2) {
@@ -919,7 +923,7 @@ MJMLX_API int mjmlx_batched_step_n_noalloc(MjmlxBatchedSim* sim, const float* ct
     int var = sim->use_gws ? step_variant(sim) : mjk::VAR_GWS;
     mjk::StepLaunch l{sim->d_kp, sim->B, 0, var, 0, ws, sim->stream, mjk::ls_cache_rows(sim->L.maxefc)};
     HIPOK(hipEventRecord(sim->ev0, sim->stream));
-    mjk::launch_step_np(sim->npset | (sim->model.nsensor > 0 ? 4 : 0), sim->nv > mjk::SPARSE_ROWS_NV, l, io, n);
+    mjk::launch_step_np(sim->npset | (sim->model.nsensor > 0 ? 4 : 0), big_kernels(sim), l, io, n);
     HIPOK(hipGetLastError());
     HIPOK(hipEventRecord(sim->ev1, sim->stream));
     sim->timed = true;

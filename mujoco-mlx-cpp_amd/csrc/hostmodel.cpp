@@ -161,6 +161,11 @@ Blob build_blob(const Model& m, std::vector<CollisionPair>* pairs_out) {
   std::vector<int> depth(nb, 0);
   int maxd = 0;
   for (int b = 1; b < nb; b++) { depth[b] = depth[m.body_parentid[b]] + 1; maxd = std::max(maxd, depth[b]); }
+  std::vector<int> level_adr(maxd + 1, 0), level_body;
+  for (int lv = 1; lv <= maxd; lv++) {
+    for (int b = 1; b < nb; b++) if (depth[b] == lv) level_body.push_back(b);
+    level_adr[lv] = (int)level_body.size();
+  }
   // last dof of each body's kinematic chain (-1: none)
   std::vector<int> lastdof(nb, -1);
   for (int b = 1; b < nb; b++) {
@@ -350,6 +355,12 @@ Blob build_blob(const Model& m, std::vector<CollisionPair>* pairs_out) {
       for (int k = 0; k < 3; k++) { r[16 + k] = fb(m.jnt_pos[3 * ja + k]); r[20 + k] = fb(m.jnt_axis[3 * ja + k]); }
     }
   }
+  std::vector<int> level_rec(level_body.size() * LEVEL_REC, 0);
+  for (size_t i = 0; i < level_body.size(); i++) {
+    int *r = &level_rec[i * LEVEL_REC], b = level_body[i];
+    const int* p = &body_rec[(size_t)b * BODY_REC];
+    r[0] = b; r[1] = p[0]; r[2] = p[1]; r[3] = p[2]; r[4] = p[23]; r[5] = p[7];
+  }
   for (int j = 0; j < m.njnt; j++) {
     int* r = &jnt_rec[(size_t)j * JNT_REC];
     for (int k = 0; k < 3; k++) { r[k] = fb(m.jnt_pos[3 * j + k]); r[4 + k] = fb(m.jnt_axis[3 * j + k]); }
@@ -412,6 +423,7 @@ Blob build_blob(const Model& m, std::vector<CollisionPair>* pairs_out) {
   std::vector<float> subtreemass = tof(m.body_subtreemass);
 #define ADDP(field, vec) d.field = reinterpret_cast<decltype(d.field)>(B.add(vec))
   ADDP(body_rootid, m.body_rootid); ADDP(body_subtree_end, send); ADDP(body_lastdof, lastdof);
+  ADDP(level_adr, level_adr); ADDP(level_rec, level_rec);
   ADDP(body_ipos, tof(m.body_ipos)); ADDP(body_iquat, tof(m.body_iquat)); ADDP(body_mass, tof(m.body_mass));
   ADDP(body_inertia, tof(m.body_inertia));
   ADDP(body_subtreemass, subtreemass); ADDP(body_invweight0, tof(m.body_invweight0));
