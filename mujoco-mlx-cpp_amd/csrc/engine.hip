@@ -778,11 +778,12 @@ MJMLX_API MjmlxBatchedSim* mjmlx_batched_create(const MjmlxModel* model, const M
     // models of at most 8 dofs, at 256 registers: measured faster than every
     // 64-lane variant on hinge chains of 2-8 dofs, slower from 16 dofs on
     // (quadruped 0.6x, humanoid 0.45x: half the waves per CU at the same LDS
-    // occupancy). MJMLX_HIP_LANES=32 or 64 forces either; the autotuner
-    // times both.
+    // occupancy), and with more bodies than lanes (two chains of 24 bodies, 8
+    // dofs, 64 envs: 0.39 ms per control step, on 64 lanes 0.23).
+    // MJMLX_HIP_LANES=32 or 64 forces either; the autotuner times both.
     s->half_ok = s->nv <= mjk::SPARSE_ROWS_NV && 2 * s->lds_bytes <= (size_t)prop.sharedMemPerBlock &&
                  2 * s->lds_bytes <= lds_max;
-    s->half = !use_gws && s->half_ok && s->nv <= 8;
+    s->half = !use_gws && s->half_ok && s->nv <= 8 && s->nb <= 32;
     if (const char* v = std::getenv("MJMLX_HIP_LANES")) s->half = !use_gws && s->half_ok && std::atoi(v) == 32;
     if (s->half) {
       s->big_regs = false;

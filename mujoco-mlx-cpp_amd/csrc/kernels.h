@@ -394,15 +394,14 @@ KDEV BodyRec body_rec(const DModel& m, int b) {
 // and working at that body's level. Beyond, the level's own, with what the stages
 // read of them in level order: looking at all bodies at every level loads
 // levels x bodies / lanes records and runs bodies of a level that share a lane
-// one after the other (64 envs, per control step: 4 chains of 20 bodies 0.39 ms so,
-// 0.33 by lists; on 32 lanes 2 chains of 24 bodies 0.39 and 0.34). The small
-// models' 64-lane kernels are without the lists, whose code costs 16384
-// quadrupeds 1 %: models of more than 64 bodies run in the kernels for any size.
-enum { LEVEL_LISTS = MJK_BIG || WAVE < 64 };
+// one after the other (64 envs, 4 chains of 20 bodies: 0.39 ms per control step
+// so, 0.33 by lists). The small models' kernels are without the lists, whose code
+// costs 16384 quadrupeds 1 % and 16384 arms 2 %: models of more than 64 bodies run
+// in the kernels for any size, of more than 32 on 64 lanes unless told otherwise.
 struct LevelBodies { const MJK_G int* rec; int n; };
 KDEV LevelBodies level_bodies(const DModel& m, int lv) {
   LevelBodies lb = {nullptr, m.nbody};
-  if (LEVEL_LISTS && m.nbody > WAVE) {
+  if (MJK_BIG && m.nbody > WAVE) {
     int a = m.level_adr[lv];
     lb.rec = m.level_rec + LEVEL_REC * a;
     lb.n = m.level_adr[lv + 1] - a;
@@ -410,7 +409,7 @@ KDEV LevelBodies level_bodies(const DModel& m, int lv) {
   return lb;
 }
 KDEV BodyRec level_body(const DModel& m, const LevelBodies& lb, const BodyRec& own, int lv, int i, int& b) {
-  if (LEVEL_LISTS && lb.rec) {
+  if (MJK_BIG && lb.rec) {
     ki4 u = kld4(lb.rec + LEVEL_REC * i), v = kld4(lb.rec + LEVEL_REC * i + 4);
     b = u[0];
     BodyRec r;
