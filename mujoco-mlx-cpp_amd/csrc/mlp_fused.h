@@ -290,8 +290,8 @@ __device__ __forceinline__ float wg_update(const WgArgs& A, size_t i, float gi) 
   return pi;
 }
 
-// One 16 x 32 tile of a weight gradient per workgroup (240 for 195-256-256-18:
-// one per CU): each wave forms the sums of its slices of K, 4 K steps of loads
+// One 16 x 32 tile of a weight gradient per workgroup (256 for 195-256-256-18,
+// one per CU, and 68 of bias columns after them): each wave forms the sums of its slices of K, 4 K steps of loads
 // ahead of the products, and leaves them in LDS, where a thread per entry adds
 // the slices in order and applies the update; no partial tile goes through
 // memory. Column tiles are the fastest index, so that an XCD (workgroup index
