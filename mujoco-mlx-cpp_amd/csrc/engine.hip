@@ -125,6 +125,7 @@ struct MjmlxData {
   int unused;
 };
 
+enum { RAYS_ONE_COPY = 256 << 10 };
 struct MjmlxBatchedSim {
   mjh::Model model;
   mjh::Blob blob;
@@ -202,6 +203,7 @@ struct MjmlxBatchedSim {
   float *d_rays = nullptr, *d_rdist = nullptr;
   int *d_rgid = nullptr, *d_gmask = nullptr;
   size_t ray_cap = 0;
+  std::vector<float> h_rays;  // both arrays of a small scan (at most RAYS_ONE_COPY bytes)
   // scratch host buffers for dumps
   float *d_dump1 = nullptr, *d_dump2 = nullptr;
   size_t dump_cap = 0;
@@ -1165,8 +1167,19 @@ MJMLX_API int mjmlx_batched_raycast(MjmlxBatchedSim* s, const float* pnt, const 
     float *d_pnt = s->d_rays, *d_vec = d_pnt + total * 3;
     // the queued steps finish before the host buffers are reused
     HIPOK(hipStreamSynchronize(s->stream));
-    HIPOK(hipMemcpyAsync(d_pnt, pnt, total * 3 * sizeof(float), hipMemcpyHostToDevice, s->stream));
-    HIPOK(hipMemcpyAsync(d_vec, vec, total * 3 * sizeof(float), hipMemcpyHostToDevice, s->stream));
+    // a few rays: both arrays in one copy, whose start costs more than moving them
+    // together (200 envs x 30 rays, 144 KB: 75 us in two, 69 in one; 500 x 64,
+    // 768 KB: 99 in two, 109 in one)
+    size_t bytes = total * 3 * sizeof(float);
+    if (2 * bytes <= RAYS_ONE_COPY) {
+      s->h_rays.resize(total * 6);
+      std::memcpy(s->h_rays.data(), pnt, bytes);
+      std::memcpy(s->h_rays.data() + total * 3, vec, bytes);
+      HIPOK(hipMemcpyAsync(d_pnt, s->h_rays.data(), 2 * bytes, hipMemcpyHostToDevice, s->stream));
+    } else {
+      HIPOK(hipMemcpyAsync(d_pnt, pnt, bytes, hipMemcpyHostToDevice, s->stream));
+      HIPOK(hipMemcpyAsync(d_vec, vec, bytes, hipMemcpyHostToDevice, s->stream));
+    }
     HIPOK(hipMemcpyAsync(s->d_gmask, mask.data(), mask.size() * sizeof(int), hipMemcpyHostToDevice, s->stream));
     if (s->use_gws)
       hipLaunchKernelGGL(k_raycast<1>, dim3(s->B), dim3(64), 0, s->stream, s->dm, s->L, s->d_qpos, s->d_rand,
