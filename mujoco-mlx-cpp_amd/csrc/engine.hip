@@ -356,6 +356,14 @@ int step_variant(const MjmlxBatchedSim* s) {
 // ones take, or more bodies than lanes (LevelBodies)
 bool big_kernels(const MjmlxBatchedSim* s) { return s->nv > mjk::SPARSE_ROWS_NV || s->nb > 64; }
 
+// step_variant for the launch: small models with elliptic cones have kernels with
+// the register routines, except at 168 VGPRs and on 32 lanes
+int launch_variant(const MjmlxBatchedSim* s) {
+  int v = step_variant(s);
+  bool regs = v == mjk::VAR_LDS || v == mjk::VAR_GWS || v == mjk::VAR_LDS_BIG;
+  return regs && !big_kernels(s) && s->model.cone != mjh::CONE_PYRAMIDAL ? v | mjk::VAR_CONES : v;
+}
+
 // one workgroup (one wave) per env: the kernel variant for the workspace
 // placement (device memory, LDS at three, two or one waves per SIMD), compiled
 // for the model's narrow-phase set and, with sensors, the sensor stage
@@ -368,7 +376,7 @@ void launch_step(MjmlxBatchedSim* s, mjk::StepIO io, int nsub) {
     mjk::launch_step_np(s->npset, true, c, io, nsub);
     io.redo_pass = 2;
   }
-  mjk::StepLaunch l{s->d_kp, s->B, 0, step_variant(s), s->lds_bytes, s->d_gws, s->stream,
+  mjk::StepLaunch l{s->d_kp, s->B, 0, launch_variant(s), s->lds_bytes, s->d_gws, s->stream,
                     mjk::ls_cache_rows(s->L.maxefc)};
   mjk::launch_step_np(s->npset | (s->model.nsensor > 0 ? 4 : 0), big_kernels(s), l, io, nsub);
 }
@@ -924,6 +932,7 @@ MJMLX_API int mjmlx_batched_step_n_noalloc(MjmlxBatchedSim* sim, const float* ct
     upload_ctrl(sim, ctrl);
     mjk::StepIO io = make_io(sim, nullptr, nullptr);
     int var = sim->use_gws ? step_variant(sim) : mjk::VAR_GWS;
+    var |= launch_variant(sim) & mjk::VAR_CONES;  // the arithmetic of the sim's own step
     mjk::StepLaunch l{sim->d_kp, sim->B, 0, var, 0, ws, sim->stream, mjk::ls_cache_rows(sim->L.maxefc)};
     HIPOK(hipEventRecord(sim->ev0, sim->stream));
     mjk::launch_step_np(sim->npset | (sim->model.nsensor > 0 ? 4 : 0), big_kernels(sim), l, io, n);

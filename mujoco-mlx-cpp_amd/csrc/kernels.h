@@ -893,8 +893,8 @@ KDEV int smooth_solve_regs(int nv, const float* A, float* x) {
 // Newton models of 21 to 32 dofs with elliptic cones; the factor of qM itself is
 // CG's preconditioner, and pyramidal models keep the rounding of the level sums
 // (newton_direction says why). Smaller models keep the levels: unrefined, the
-// register solve had 1.12 (12 dofs) to 1.23 times (20) their error. REGS: not
-// the 168-VGPR kernels.
+// register solve had 1.12 (12 dofs) to 1.23 times (20) their error. REGS: as in
+// newton_direction.
 template <bool REGS>
 KDEV bool solve_in_regs(const DModel& m) { return REGS && m.solver == 2 && m.cone != 0 && m.nv > 20; }
 #else
@@ -3326,15 +3326,17 @@ KDEV void newton_solve(const DModel& m, const Layout& L, float* w) {
 // solve in registers), 18 of 491520 implicitfast quadrupeds ended more than
 // 8e-4 of the RMS velocity away after 4 substeps (up to 2e-2), with the updates
 // none; of 5.6 million humanoids none either way.
-// The 168-VGPR kernels (TRI_CACHE false) have the workspace's factor only: with
-// the register routines compiled in they spill (16384 quadrupeds, which never
-// call them, 3.39 ms per control step against 3.22 without).
-template <bool TRI_CACHE>
+// REGS: the kernels of their own that elliptic models take. Compiled into the
+// others' the register routines cost those that never call them: 16384 quadrupeds
+// 3.39 ms per control step against 3.22 without (168 VGPRs: spills), 4 boxes
+// under CG, 100 / 500 envs 1.145 / 1.20 ms against 1.10 / 1.16 (scalar spills,
+// 155 -> 435).
+template <bool TRI_CACHE, bool REGS>
 KDEV int newton_direction(const DModel& m, const Layout& L, float* w, int nefc, bool refactor, int nch,
                           const unsigned long long* chmask, KProfAcc* pa) {
   int st = 0;
 #if WAVE == 64 && !MJK_BIG
-  if (TRI_CACHE && m.cone != 0) {
+  if (REGS && m.cone != 0) {
     int nv = m.nv, nrow = cone_virtual_rows(m, L, w, nefc);
     if (nrow >= 0) {
       float* A = w + L.H;
@@ -3734,7 +3736,7 @@ KDEV float linesearch_(const DModel& m, const Layout& L, float* w, int nefc, int
 // termination test, qfrc_constraint = J^T force.
 // pred: the learned warm-start candidate (the env's row of the prediction in
 // device memory), or null
-template <bool TRI_CACHE>
+template <bool TRI_CACHE, bool REGS>
 KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KProfAcc* pa, const float* pred,
                   LsCache lc) {
   int* misc = iptr(w, L.misc);
@@ -3785,7 +3787,7 @@ KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KP
   const float* Jv = w + L.efc_Jv;
   KPROF_MARK(pa, KP_SOLVE_INIT);
   if (newton) {
-    st |= newton_direction<TRI_CACHE>(m, L, w, nefc, true, 0, nullptr, pa);
+    st |= newton_direction<TRI_CACHE, REGS>(m, L, w, nefc, true, 0, nullptr, pa);
     KPROF_MARK(pa, KP_NSOLVE);
   } else {
     for (int i = LANE; i < nv; i += WAVE) Mg[i] = grad[i];
@@ -3799,7 +3801,7 @@ KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KP
     int exact = 0;
     KPROF_MARK(pa, KP_DIR);
     float dec = 0.f;
-    float alpha = linesearch<TRI_CACHE>(kfresh(m), kfresh(L), w, nefc, &exact, newton ? nullptr : &dec, lc,
+    float alpha = linesearch<WAVE == 64 && !MJK_BIG ? REGS : TRI_CACHE>(kfresh(m), kfresh(L), w, nefc, &exact, newton ? nullptr : &dec, lc,
                              newton ? &cost : nullptr);
     KPROF_MARK(pa, KP_LS);
     *niter_out = it + 1;
@@ -3830,7 +3832,7 @@ KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KP
       // H depends on qacc only through the active set. (One call for both this
       // direction and the first one, at the loop's head, costs the stored
       // factor's kernels: 16384 quadrupeds 3.07 -> 3.19 ms, 64 399 -> 413 us.)
-      st |= newton_direction<TRI_CACHE>(kfresh(m), kfresh(L), w, nefc, false, nch, chm, pa);
+      st |= newton_direction<TRI_CACHE, REGS>(kfresh(m), kfresh(L), w, nefc, false, nch, chm, pa);
       KPROF_MARK(pa, KP_NSOLVE);
       for (int i = LANE; i < nv; i += WAVE) srch[i] = -Mg[i];
     } else {
@@ -3862,7 +3864,7 @@ KDEV int st_solve(const DModel& m, const Layout& L, float* w, int* niter_out, KP
 // Euler (implicit dof damping when present) / implicitfast, then the position
 // update; free and ball quaternions are integrated in FP64
 // (reference euler.hpp:26-110 restated with MuJoCo's mj_integratePos).
-template <bool DENSE>
+template <bool DENSE, bool REGS>
 KDEV int st_integrate(const DModel& m, const Layout& L, float* w) {
   int nv = m.nv;
   float *qvel = w + L.qvel, *qpos = w + L.qpos, *qacc = w + L.qacc, *ws = w + L.qacc_ws;
@@ -3895,7 +3897,7 @@ KDEV int st_integrate(const DModel& m, const Layout& L, float* w) {
     const float *qfs = w + L.qfrc_smooth, *qfc = w + L.qfrc_constraint;
     for (int k = LANE; k < nv; k += WAVE) acc[k] = qfs[k] + qfc[k];
     KSYNC();
-    if (solve_in_regs<DENSE>(m)) {
+    if (solve_in_regs<REGS>(m)) {
       st |= smooth_solve_regs(nv, Bm, acc);
     } else {
       st |= factor_ld<DENSE>(m, Bm, A);
@@ -4269,7 +4271,8 @@ KDEV void write_features(const DModel& m, const Layout& L, const float* w, float
 // NPSET: bits 0-1 the narrow-phase set (0 basic pairs, 1 + capsule-box /
 // box-box, 2 + GJK/EPA), bit 2 the sensor stage (models with sensors only, so
 // the plain step carries none of its code), bit 3 set by the register-capped
-// kernel variant
+// kernel variant, bit 6 the register routines of elliptic models (small models'
+// 64-lane kernels other than the register-capped one)
 // m and L: the sim's device-memory copy (KParams), read through kfresh().
 // lc: LDS for the line search's rows beside a device-memory workspace (or none)
 template <int NPSET>
@@ -4300,9 +4303,9 @@ KDEV void run_env(const DModel& m, const Layout& L, float* w, const StepIO& io, 
     st_kinematics(m, L, w);
     st_com_pos(m, L, w);
     st_crb(m, L, w);
-    if (nv > 0 && (!solve_in_regs<(NPSET & 8) == 0>(m) || io.dump1)) factor_ld<(NPSET & 8) == 0>(m, w + L.qM, w + L.qLD);
+    if (nv > 0 && (!solve_in_regs<(NPSET & 64) != 0>(m) || io.dump1)) factor_ld<(NPSET & 8) == 0>(m, w + L.qM, w + L.qLD);
     st_com_vel(m, L, w);
-    st_smooth<(NPSET & 8) == 0>(m, L, w);
+    st_smooth<(NPSET & 64) != 0>(m, L, w);
     // the kinematics and dynamics intermediates are intact only here: the
     // constraint rows of a full substep take their space
     dump_ws(L, w, io.dump1, env);
@@ -4325,11 +4328,11 @@ KDEV void run_env(const DModel& m, const Layout& L, float* w, const StepIO& io, 
     st_crb(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_CRB);
     // a dump shows qM's factor also where the solves do without it
-    if (nv > 0 && (!solve_in_regs<(NPSET & 8) == 0>(m) || (last && io.dump1))) st |= factor_ld<(NPSET & 8) == 0>(kfresh(m), w + L.qM, w + L.qLD);
+    if (nv > 0 && (!solve_in_regs<(NPSET & 64) != 0>(m) || (last && io.dump1))) st |= factor_ld<(NPSET & 8) == 0>(kfresh(m), w + L.qM, w + L.qLD);
     KPROF_MARK(&pa, KP_FACTOR);
     st_com_vel(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_COMVEL);
-    st |= st_smooth<(NPSET & 8) == 0>(kfresh(m), kfresh(L), w);
+    st |= st_smooth<(NPSET & 64) != 0>(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_SMOOTH);
     if (last && io.has_aux) write_aux(m, L, w, io.aux, env);
     if constexpr ((NPSET & 4) != 0)
@@ -4346,12 +4349,12 @@ KDEV void run_env(const DModel& m, const Layout& L, float* w, const StepIO& io, 
     }
     if (last) dump_ws(L, w, io.dump1, env);
     int it = 0;
-    st |= st_solve<(NPSET & 8) == 0>(kfresh(m), kfresh(L), w, &it, &pa,
+    st |= st_solve<(NPSET & 8) == 0, (NPSET & 64) != 0>(kfresh(m), kfresh(L), w, &it, &pa,
                                      io.qacc_pred && s == 0 ? io.qacc_pred + (size_t)env * nv : nullptr, lc);
     niter += it;
     if (last && io.has_aux) write_cfrc_ext(m, L, w, io.aux, env, true);
     if (last) dump_ws(L, w, io.dump2, env);
-    st |= st_integrate<(NPSET & 8) == 0>(kfresh(m), kfresh(L), w);
+    st |= st_integrate<(NPSET & 8) == 0, (NPSET & 64) != 0>(kfresh(m), kfresh(L), w);
     KPROF_MARK(&pa, KP_INTEGRATE);
   }
   int bad = 0;

@@ -22,7 +22,9 @@ enum {
   VAR_GWS_OCC = 4,  // device memory, 168 VGPRs
   VAR_LDS_HALF = 5,      // LDS, 32 lanes per env (two envs per wave), 256 registers
   VAR_LDS_OCC_HALF = 6,  // LDS, 32 lanes per env, 168 VGPRs
-  VAR_N = 7
+  VAR_N = 7,
+  // added to VAR_LDS, VAR_GWS or VAR_LDS_BIG: small models with elliptic cones
+  VAR_CONES = 64
 };
 
 struct StepLaunch {

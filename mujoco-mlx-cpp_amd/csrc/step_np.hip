@@ -117,6 +117,20 @@ void MJK_LAUNCH(const StepLaunch& l, const StepIO& io, int nsub) {
   bool gws = l.variant == VAR_GWS || l.variant == VAR_GWS_OCC;
   // device-memory workspaces: the dynamic LDS holds the line search's row cache
   size_t sh = gws ? (size_t)l.ls_cap * sizeof(LsRow4) : l.lds_bytes;
+#if !MJK_BIG
+  // bit 64 of the set names the kernels with the register routines of elliptic models
+  switch (l.variant) {
+    case VAR_GWS | VAR_CONES:
+      hipLaunchKernelGGL((k_step<NP | 64, 1>), g, b, (size_t)l.ls_cap * sizeof(LsRow4), l.stream, l.kp, io, l.B, l.env0, nsub, l.gws, l.ls_cap);
+      return;
+    case VAR_LDS_BIG | VAR_CONES:
+      hipLaunchKernelGGL((k_step_big<NP | 64>), g, b, l.lds_bytes, l.stream, l.kp, io, l.B, l.env0, nsub);
+      return;
+    case VAR_LDS | VAR_CONES:
+      hipLaunchKernelGGL((k_step<NP | 64, 0>), g, b, l.lds_bytes, l.stream, l.kp, io, l.B, l.env0, nsub, l.gws, 0);
+      return;
+  }
+#endif
   switch (l.variant) {
     case VAR_GWS_OCC:
       hipLaunchKernelGGL((k_step_occ<NP, 1>), g, b, sh, l.stream, l.kp, io, l.B, l.env0, nsub, l.gws, l.ls_cap);

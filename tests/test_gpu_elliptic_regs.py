@@ -38,11 +38,11 @@ def test_smooth(nv, monkeypatch):
     smooth.test_chain(nv)
 
 
-@pytest.mark.parametrize("variant", [0, 2, 3])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3])
 def test_register_budgets(variant):
-    """Humanoids under every register budget of the 64-lane kernels (168 VGPRs:
-    contacts read per evaluation, factors in the workspace), to the bars of the
-    humanoid's parity test."""
+    """Humanoids under every register budget of the 64-lane kernels and from device
+    memory (168 VGPRs: contacts read per evaluation, factors in the workspace), to
+    the bars of the humanoid's parity test."""
     model = capi.Model(scenes.humanoid_xml())
     B = 24
     q, qv, qa, ctrl, orc = humanoid._states(model, B, 4)
